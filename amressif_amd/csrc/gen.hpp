@@ -63,8 +63,7 @@ struct Ctx {
     int64_t npartials = 0;
     int nb_face[3]{};        // blocks per face direction in k_gen_update
     int last_P = 8, last_V = 8;
-    int flux_z = 1;          // 3D: fluxTotal by the z-march kernel (0: one thread per cell)
-    int flux_zc = 16;        // z-march kernel: planes per workgroup
+    int s3_ntx = 0, s3_nty = 0, s3_zc = 0;  // 3D stage: tiles in x and y, planes per workgroup
 };
 
 // ---- launchers (kernels_gen.hip); every guarded kernel returns at once once
@@ -74,6 +73,12 @@ hipError_t flux(const Ctx &c, hipStream_t s, double *const *faces, const double 
 // stage update of every face: u* <- u^k + rk (R - c15 u* + C); last: the
 // norm partials of u^k - u* and u^k <- u* as well
 hipError_t update(const Ctx &c, hipStream_t s, double rk, int last, const Ctl *guard);
+// 3D: one RK4 stage in one pass, out <- base + rk (R(in) - c15 in + C); out
+// aliases neither in nor base.  last: the norm partials of base - out as well
+hipError_t stage3(const Ctx &c, hipStream_t s, double *const *in, double *const *base, double *const *out, double rk,
+                  int last, const Ctl *guard);
+void stage3_shape(int n, int *ntx, int *nty, int *zc);
+int stage3_blocks(const Ctx &c);
 hipError_t fin_pseudo(const Ctx &c, hipStream_t s, Ctl *ctl);
 hipError_t bdf2(const Ctx &c, hipStream_t s);
 // b = (1.5/dt) D(faces) (b may be null: the norm only); partials of max|D|, sum b

@@ -177,8 +177,6 @@ int amr_gen_create(amressif_ctx *ctx)
     if (in.poisson_solver != 0)
         return gfail(ctx, AMRESSIF_ERR_UNSUPPORTED, "3D and periodic runs use the multigrid Poisson solve");
     auto *gp = new G::Ctx();
-    if (const char *e = std::getenv("AMRESSIF_GEN_FLUXZ")) gp->flux_z = std::atoi(e) ? 1 : 0;
-    if (const char *e = std::getenv("AMRESSIF_GEN_FZC")) gp->flux_zc = std::max(1, std::min(1024, std::atoi(e)));
     c.gen = gp;
     G::Ctx &gc = *gp;
     G::Geom &g = gc.g;
@@ -250,6 +248,10 @@ int amr_gen_create(amressif_ctx *ctx)
             return gfail(ctx, AMRESSIF_ERR_UNSUPPORTED,
                          "coarsest multigrid level above 1024 cells (n_cell = m 2^k with m^dim > 1024, m odd)");
     }
+    if (dim == 3) {
+        G::stage3_shape(n, &gc.s3_ntx, &gc.s3_nty, &gc.s3_zc);
+        if (const char *e = std::getenv("AMRESSIF_GEN_S3ZC")) gc.s3_zc = std::max(1, std::min(n + 1, std::atoi(e)));
+    }
     const size_t cellsz = (size_t)g.ncell;
 #define GALLOC(p, cnt)                                                                     \
     do {                                                                                   \
@@ -261,14 +263,15 @@ int amr_gen_create(amressif_ctx *ctx)
         GALLOC(&gc.B[d], g.nf[d]); GALLOC(&gc.S[d], g.nf[d]);
     }
     GALLOC(&gc.X, (size_t)g.xs * dim);
-    GALLOC(&gc.T, cellsz * dim);
+    if (dim == 2) GALLOC(&gc.T, cellsz * dim);
     GALLOC(&gc.p, cellsz); GALLOC(&gc.phi, cellsz); GALLOC(&gc.b, cellsz);
     for (int l = 0; l < gc.nlev; ++l) {
         GALLOC(&gc.lev[l].e, (size_t)gc.lev[l].ncell);
         GALLOC(&gc.lev[l].r, (size_t)gc.lev[l].ncell);
     }
     gc.npartials = std::max<int64_t>(2 * ((g.ncell + G::kBlock - 1) / G::kBlock),
-                                     (int64_t)gc.nb_face[0] + gc.nb_face[1] + gc.nb_face[2]) + 64;
+                                     3 * (dim == 3 ? (int64_t)G::stage3_blocks(gc)
+                                                   : (int64_t)gc.nb_face[0] + gc.nb_face[1])) + 64;
     GALLOC(&gc.partials, (size_t)gc.npartials);
     {
         std::vector<double> pinv;
@@ -545,11 +548,48 @@ int amr_gen_advance(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats)
     GCHK(amr::launch_ctl_set(c, c.in.momentum_tolerance, c.in.poisson_tol_rel, c.in.poisson_tol_abs, c.in.IterNum,
                              c.in.mg_max_iter));
     int status = AMRESSIF_OK;
+    const bool dim3 = g.dim == 3;
     for (int s = 0; s < nsteps; ++s) {
         GCHK(G::bdf2(gc, c.stream));
         GCHK(amr::launch_ctl_reset_step(c));
         // ---- momentum predictor
-        if (!g.pseudo) {
+        if (dim3) {
+            // u^{n-1}'s array is free once the constant holds it, and becomes the
+            // scratch of stages 1 and 3; stages 2 and 4 of pseudo-iteration k write
+            // the array (k odd: B, even: S) that then is the base of the next one
+            double **F[3] = {gc.Up, gc.B, gc.S};
+            auto iter_out = [&](int k) { return F[(k & 1) ? 1 : 2]; };
+            int count;
+            if (!g.pseudo) {
+                GCHK(G::stage3(gc, c.stream, gc.U, gc.U, iter_out(1), g.dt / 1.5, 1, c.ctl));
+                GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
+                count = 1;
+            } else {
+                int done = 0, batch = std::max(1, gc.last_P), k = 0;
+                while (!done) {
+                    for (int it = 0; it < batch; ++it) {
+                        double **base = k == 0 ? gc.U : iter_out(k), **out = iter_out(k + 1);
+                        GCHK(G::stage3(gc, c.stream, base, base, F[0], gc.rk[0], 0, c.ctl));
+                        GCHK(G::stage3(gc, c.stream, F[0], base, out, gc.rk[1], 0, c.ctl));
+                        GCHK(G::stage3(gc, c.stream, out, base, F[0], gc.rk[2], 0, c.ctl));
+                        GCHK(G::stage3(gc, c.stream, F[0], base, out, gc.rk[3], 1, c.ctl));
+                        GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
+                        ++k;
+                    }
+                    if (int rc = poll(ctx)) return rc;
+                    done = c.ctl_host->mom_done;
+                    batch = std::max(2, batch / 2);
+                }
+                count = std::max(1, c.ctl_host->mom_count);  // launches past it left every array as it was
+                gc.last_P = count;
+            }
+            // u* is iter_out(count)'s; u^n becomes u^{n-1}, and the projection
+            // writes u^{n+1} into the scratch
+            for (int d = 0; d < 3; ++d) {
+                if (count & 1) std::swap(gc.B[d], gc.S[d]);
+                std::swap(gc.U[d], gc.Up[d]);
+            }
+        } else if (!g.pseudo) {
             GCHK(G::cells(gc, c.stream, gc.S, gc.X, c.ctl));
             GCHK(G::flux(gc, c.stream, gc.S, gc.X, gc.T, c.ctl));
             GCHK(G::update(gc, c.stream, g.dt / 1.5, 1, c.ctl));
@@ -612,7 +652,8 @@ int amr_gen_advance(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats)
 }
 
 // ================================================================== timing
-// which: 0 cells, 1 flux, 2 stage update (the three passes of one stage)
+// which: 0 cells; 1, 2: 2D the fluxTotal and update passes of a stage, 3D the
+// whole stage without and with the norm partials
 int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, double *bytes_per_launch)
 {
     Ctx &c = ctx->c;
@@ -628,10 +669,13 @@ int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, 
         GCHK(hipMemcpyAsync(gc.B[d], gc.U[d], g.nf[d] * 8, hipMemcpyDeviceToDevice, c.stream));
     }
     GCHK(G::bdf2(gc, c.stream));
-    GCHK(G::cells(gc, c.stream, gc.S, gc.X, nullptr));
-    GCHK(G::flux(gc, c.stream, gc.S, gc.X, gc.T, nullptr));
+    if (g.dim == 2) {
+        GCHK(G::cells(gc, c.stream, gc.S, gc.X, nullptr));
+        GCHK(G::flux(gc, c.stream, gc.S, gc.X, gc.T, nullptr));
+    }
     auto launch = [&]() -> hipError_t {
-        if (which == 0) return G::cells(gc, c.stream, gc.S, gc.X, nullptr);
+        if (which == 0) return G::cells(gc, c.stream, gc.U, gc.X, nullptr);
+        if (g.dim == 3) return G::stage3(gc, c.stream, gc.U, gc.B, gc.S, gc.rk[0], which == 2, nullptr);
         if (which == 1) return G::flux(gc, c.stream, gc.S, gc.X, gc.T, nullptr);
         return G::update(gc, c.stream, 0.0, 0, nullptr);  // rk = 0: the faces keep their values
     };
@@ -647,11 +691,13 @@ int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, 
     *avg_ms = ms / reps;
     // algorithmic bytes (FP64), each array read or written once per launch:
     // cells: dim face arrays in, dim ghosted cell comps out; flux: dim face
-    // arrays and X in, T out; update: T, u*, u^k, C in, u* out
+    // arrays and X in, T out; update: T, u*, u^k, C in, u* out; the 3D stage:
+    // u*, u^k, C in, u* out
     const double faces = (double)(g.nf[0] + g.nf[1] + (g.dim == 3 ? g.nf[2] : 0));
     const double cellsd = (double)g.ncell * g.dim;
     double bytes = 0.0;
     if (which == 0) bytes = 8.0 * (faces + (double)g.xs * g.dim);
+    else if (g.dim == 3) bytes = 8.0 * 4.0 * faces;
     else if (which == 1) bytes = 8.0 * (faces + (double)g.xs * g.dim + cellsd);
     else bytes = 8.0 * (cellsd + 4.0 * faces);
     if (bytes_per_launch) *bytes_per_launch = bytes;

@@ -1,7 +1,8 @@
 // Kernels of the general path (gen.hpp): the fractional step on n^dim cells,
 // dim 2 or 3, with periodic directions beside the wall codes, FP64.
 //
-// One RK4 dual-time stage is three streaming passes:
+// One RK4 dual-time stage is one pass in 3D (k_gen_stage3) and three streaming
+// passes in 2D:
 //   k_gen_cells  : cell velocities X from the faces with every ghost layer the
 //                  stencils read (cont2cart, utilities.cpp:16-350; periodic
 //                  images and the wall rules, corners in the reference's pass
@@ -170,74 +171,391 @@ __global__ __launch_bounds__(B) void k_gen_flux(Geom g, const double *f0, const 
     }
 }
 
-// The same fluxTotal for a 3D box, marched along z: a workgroup owns a 64 x 4
-// column tile and zc planes, and each thread keeps its column's X(z - 2 ..
-// z + 2) of every component in registers (the next plane loaded one step
-// ahead), so the z-stencil reads X from memory once per cell instead of five
-// times, and the x and y neighbours of the current plane come from the
-// tile's own and its halo's loads of that plane (L1 and L2).  k_gen_flux's
-// one-thread-per-cell order reads the five planes of a cell from five
-// distant parts of X, which at 256^3 (540 KB per plane and component) do not
-// stay in an XCD's L2.  Per cell the arithmetic is k_gen_flux's, term by term.
-constexpr int kFzTX = 64, kFzTY = 4;
-__global__ __launch_bounds__(256) void k_gen_flux_z(Geom g, const double *f0, const double *f1, const double *f2,
-                                                    const double *X, double *T, const Ctl *guard, int ntx, int nty,
-                                                    int zc)
+// A face's velocity as the three factors its QUICK fluxes share: with X(-), X(+) the
+// cells at the face and D their second differences, QUICK's flux
+// vel ((X(-) + X(+))/2 - D(upwind)/8) is con (X(-) + X(+)) + cp D(-) + cm D(+).
+// kq = -1/(8 dx), so that a cell's divergence is a plain difference of fluxes.
+struct FaceVel {
+    double con, cp, cm;
+};
+__device__ __forceinline__ FaceVel face_vel(double vel, double kq)
 {
-    if (guard && guard->mom_done) return;
+    const double q = kq * vel;
+    FaceVel f;
+    f.con = -4.0 * q;
+    f.cp = fmin(q, 0.0);
+    f.cm = fmax(q, 0.0);
+    return f;
+}
+__device__ __forceinline__ double face_flux(const FaceVel &f, double xm, double xp, double dm, double dp)
+{
+    return f.con * (xm + xp) + (f.cp * dm + f.cm * dp);
+}
+
+// ------------------------------------------------ one RK4 stage in one pass (3D)
+// u* <- u^k + rk (R(u*) - (1.5/dt) u* + C) on every face, from the faces
+// alone: 96 B per cell (u*, u^k and C in, the new u* out; 72 B where u* is
+// u^k), where the three passes it replaces (cell velocities, fluxTotal, update)
+// moved 2.4 times that.  At 256^3 a launch takes 439 us (3.7 TB/s; with the norm
+// partials 449) against 162 + 390 + 374 us of the three passes, at 144^3 88 us
+// against 34 + 69 + 60, at 64^3 22 against 5.5 + 22 + 7.  Bound by the arithmetic
+// of a plane (2.7 us, about 60% of it in the FP64 pipe) more than by memory.
+//
+// A workgroup owns 58 columns x kS3Y rows and marches up a chunk of planes.  Wave r
+// works on rows y0 - 3 + 2 r and the next, lane l on column x0 - 3 + l, so the
+// stencil's three faces on either side are waves and lanes of the same workgroup:
+//  * x neighbours come from adjacent lanes (DPP);
+//  * y neighbours are the thread's other row or come through LDS: a plane's cell
+//    velocities, double-buffered, one barrier per plane.  The y-flux total T_v of
+//    the wave below takes the same barrier one plane later, so the lower row's
+//    v-faces of plane z are written at plane z + 1;
+//  * z neighbours stay in registers: cell velocities of planes z .. z + 2, the
+//    second difference and the flux at the plane's lower face.  The planes' x- and
+//    y-faces wait in an LDS ring until their plane is the march's.
+// One wait for memory per plane, at its top: for the faces of plane z + 2 and the
+// base and constant of plane z, loaded a plane ago; then the next plane's loads
+// and the last plane's results go out.  Waves with one row each (16 of them, up to
+// 128 VGPRs) had to load the base and constant in the plane that uses them: 620 us
+// at 256^3.  Planes are addressed as buffers (scalar base, 32-bit offsets): with
+// 64-bit addresses the compiler kept one per array and row in registers and
+// spilled them, and each reload waited for every load in flight (934 us).
+// A face's flux is con s + cp D(-) + cm D(+) (FaceVel): the second differences serve
+// QUICK on both sides of a cell and the Laplacian.
+// Ghosts: periodic directions wrap a load's index; past a wall it is mirrored
+// (face -q for q < 0, 2n - q for q > n: the average of a ghost cell's two faces is
+// then its mirror cell's) and the cell takes the wall's rule, affine in the mirror
+// cell: sg X + ct.  The output must not alias the stencil input.
+// One workgroup per CU; the chunk of planes is chosen on the host so that the grid
+// fills the CUs in whole rounds (stage3_shape).
+typedef unsigned Dwords2 __attribute__((ext_vector_type(2)));
+constexpr int kS3X = 58, kS3W = 8, kS3Y = 2 * kS3W - 5;
+struct Stage3 {
+    const double *s[3], *b[3], *c[3];
+    double *o[3];
+    double *partials;
+    double rk;
+    double kq[3], kv[3];        // -1/(8 dx), 1/(dx^2 Re)
+    double sg[6][3], ct[6][3];  // wall rules: sides W, E, S, N, B, F
+    int ntx, nty, zc;
+};
+
+template <bool LAST>
+__global__ __launch_bounds__(64 * kS3W) void k_gen_stage3(Geom g, Stage3 a, const Ctl *guard)
+{
+    __shared__ double shX[2][3][2 * kS3W][64];
+    __shared__ double shT[2][kS3W][64];
+    __shared__ double shF[4][2][2 * kS3W][64];  // x- and y-faces of planes z .. z + 2 (slot: plane mod 4)
+    // the rules in LDS: only edge waves and planes use them, and as kernel arguments
+    // they would hold 72 scalar registers through the march
+    __shared__ double shR[6][3][2];
+    if (guard && guard->mom_done) return;  // the same for every thread of the launch
+    const int n = g.n, lane = threadIdx.x & 63;
+    const int r = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int blk = xcd_block(blockIdx.x, gridDim.x);
-    const int tx = blk % ntx, ty = (blk / ntx) % nty, tz = blk / (ntx * nty);
-    const int n = g.n;
-    const int x = tx * kFzTX + (int)(threadIdx.x & 63), y = ty * kFzTY + (int)(threadIdx.x >> 6);
-    const int z0 = tz * zc, z1 = min(z0 + zc, n);
-    if (x >= n || y >= n || z0 >= n) return;  // no barrier below: a thread past the edge just ends
-    const int64_t s = n + 4, sz = s * s, xs = g.xs;
-    int64_t xc = xidx(g, x, y, z0);
-    double w[3][5];  // X(x, y, z - 2 .. z + 2) per component
+    const int tx = blk % a.ntx, ty = (blk / a.ntx) % a.nty, tz = blk / (a.ntx * a.nty);
+    const int x0 = tx * kS3X - 3, i = x0 + lane, y = ty * kS3Y + 2 * r - 3;  // column, lower row
+    const int z0 = tz * a.zc, z1 = min(z0 + a.zc, n + 1);  // face planes z0 .. z1 - 1 (plane n: z-faces only)
+    const bool px = g.per[0], py = g.per[1], pz = g.per[2];
+    if (threadIdx.x < 18) {
+        shR[threadIdx.x / 3][threadIdx.x % 3][0] = a.sg[threadIdx.x / 3][threadIdx.x % 3];
+        shR[threadIdx.x / 3][threadIdx.x % 3][1] = a.ct[threadIdx.x / 3][threadIdx.x % 3];
+    }
+    __syncthreads();
+    auto cell_of = [n](int q, bool per) {  // -3 <= q; past n + 2: any cell (nothing that is kept reads it)
+        q = min(q, n + 2);
+        if (per) return q < 0 ? q + n : (q >= n ? q - n : q);
+        return q < 0 ? -1 - q : (q >= n ? 2 * n - 1 - q : q);
+    };
+    auto face_of = [n](int q, bool per) {  // periodic: face n keeps its own copy of face 0
+        q = min(q, n + 3);
+        if (per) return q < 0 ? q + n : (q > n ? q - n : q);
+        return q < 0 ? -q : (q > n ? 2 * n - q : q);
+    };
+    const unsigned su = (unsigned)(n + 1) * n, sw = (unsigned)n * n;  // plane strides (x- and y-faces alike; z-faces)
+    // byte offsets in a plane: x- and z-faces of the two rows, y-faces of the three; on
+    // output rows and lanes they are the thread's own faces
+    unsigned ou[2], oc[2], ov[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
+    for (int q = 0; q < 2; ++q) {
+        ou[q] = 8u * (unsigned)(face_of(i, px) + (n + 1) * cell_of(y + q, py));
+        oc[q] = 8u * (unsigned)(cell_of(i, px) + n * cell_of(y + q, py));
+    }
 #pragma unroll
-        for (int k = 0; k < 5; ++k) w[c][k] = X[c * xs + xc + (k - 2) * sz];
-    double fzl = f2[fidx(g, 2, x, y, z0)], fzh = f2[fidx(g, 2, x, y, z0 + 1)];
-    for (int z = z0; z < z1; ++z) {
-        double nw[3] = {0.0, 0.0, 0.0}, nfz = 0.0;
-        if (z + 1 < z1) {  // the next step's new plane z + 3 (a ghost plane at most) and z-face z + 2
+    for (int q = 0; q < 3; ++q) ov[q] = 8u * (unsigned)(cell_of(i, px) + n * face_of(y + q, py));
+    // a plane of `count` doubles as a buffer resource: a scalar base and 32-bit byte
+    // offsets (64-bit addresses would be kept in registers per array), and an access
+    // past it reads 0 or writes nothing, so that masks are offsets
+    auto plane = [](const double *base, unsigned first, unsigned count) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(base + first), 0, 8 * count, 0x00020000);
+    };
+    auto ld = [](__amdgpu_buffer_rsrc_t p, unsigned off) {
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(p, off, 0, 0));
+    };
+    auto st = [](__amdgpu_buffer_rsrc_t p, unsigned off, double v) {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(Dwords2, v), p, off, 0, 0);
+    };
+    auto rule = [&](int side, double *X) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) nw[c] = X[c * xs + xc + 3 * sz];
-            nfz = f2[fidx(g, 2, x, y, z + 2)];
+        for (int c = 0; c < 3; ++c) X[c] = shR[side][c][0] * X[c] + shR[side][c][1];
+    };
+    const bool xedge = !px && (x0 < 0 || x0 + 63 >= n), yedge = !py && (y < 0 || y + 1 >= n);
+    struct Plane {  // x-faces and y-faces of one plane, z-faces above it
+        double u[2], v[3], w[2];
+    };
+    auto load = [&](int z, Plane &P) {
+        const auto u = plane(a.s[0], cell_of(z, pz) * su, su), v = plane(a.s[1], cell_of(z, pz) * su, su),
+                   w = plane(a.s[2], face_of(z + 1, pz) * sw, sw);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            P.u[q] = ld(u, ou[q]);
+            P.w[q] = ld(w, oc[q]);
         }
-        const double fw0 = f0[fidx(g, 0, x, y, z)], fe0 = f0[fidx(g, 0, x + 1, y, z)];
-        const double fw1 = f1[fidx(g, 1, x, y, z)], fe1 = f1[fidx(g, 1, x, y + 1, z)];
-        const int64_t q = cidx(g, x, y, z);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const double *Xc = X + c * xs + xc;
-            const double C = w[c][2];
-            double m2 = Xc[-2], m1 = Xc[-1], p1 = Xc[1], p2 = Xc[2];
-            double Fw = quick(fw0, m2, m1, C, p1), Fe = quick(fe0, m1, C, p1, p2);
-            double conv = (Fe - Fw) * g.idx[0];
-            const double l0 = (p1 - 2.0 * C + m1) * g.idx2[0];
-            m2 = Xc[-2 * s]; m1 = Xc[-s]; p1 = Xc[s]; p2 = Xc[2 * s];
-            Fw = quick(fw1, m2, m1, C, p1);
-            Fe = quick(fe1, m1, C, p1, p2);
-            conv = conv + (Fe - Fw) * g.idx[1];
-            const double l1 = (p1 - 2.0 * C + m1) * g.idx2[1];
-            m2 = w[c][0]; m1 = w[c][1]; p1 = w[c][3]; p2 = w[c][4];
-            Fw = quick(fzl, m2, m1, C, p1);
-            Fe = quick(fzh, m1, C, p1, p2);
-            conv = conv + (Fe - Fw) * g.idx[2];
-            const double l2 = (p1 - 2.0 * C + m1) * g.idx2[2];
-            double visc = (l0 + l1) * g.iren;
-            visc = visc + l2 * g.iren;
-            T[q + (int64_t)c * g.ncell] = (0.0 - conv) + visc;
+        for (int q = 0; q < 3; ++q) P.v[q] = ld(v, ov[q]);
+    };
+    // cell velocities of plane z from its faces and the z-faces below it
+    auto cells = [&](int z, const Plane &P, const double *wl, double (*X)[3]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            X[q][0] = 0.5 * (P.u[q] + lane_next(P.u[q]));
+            X[q][1] = 0.5 * (P.v[q] + P.v[q + 1]);
+            X[q][2] = 0.5 * (wl[q] + P.w[q]);
+        }
+        if (xedge) {
+            if (i < 0) {
+                rule(0, X[0]);
+                rule(0, X[1]);
+            } else if (i >= n) {
+                rule(1, X[0]);
+                rule(1, X[1]);
+            }
+        }
+        if (yedge) {
+            if (y < 0) rule(2, X[0]);
+            if (y >= n) rule(3, X[0]);
+            if (y + 1 < 0) rule(2, X[1]);
+            if (y + 1 >= n) rule(3, X[1]);
+        }
+        if (!pz && (z < 0 || z >= n)) {
+            rule(z < 0 ? 4 : 5, X[0]);
+            rule(z < 0 ? 4 : 5, X[1]);
+        }
+    };
+    auto keep = [&](int z, const Plane &P) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            shF[z & 3][0][2 * r + q][lane] = P.u[q];
+            shF[z & 3][1][2 * r + q][lane] = P.v[q];
+        }
+    };
+    // output rows 3 .. 2 kS3W - 3 of the workgroup's: both rows of waves 2 .. kS3W - 2, wave 1's upper one
+    const bool rowT = r >= 1 && r <= kS3W - 2;
+    const bool lanO = rowT && lane >= 3 && lane <= 60;
+    unsigned fu[2], fv[2], fw[2];  // the faces this thread updates: their offsets, or past the plane
+    constexpr unsigned kNone = 0x80000000u;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const bool o = lanO && (q == 1 || r >= 2);
+        fu[q] = o && y + q < n && i <= n ? ou[q] : kNone;
+        fv[q] = o && y + q <= n && i < n ? ov[q] : kNone;
+        fw[q] = o && y + q < n && i < n ? oc[q] : kNone;
+    }
+    struct Upd {  // base and constant of the three faces of both rows
+        double ub[2], uc[2], vb[2], vc[2], wb[2], wc[2];
+    };
+    auto load_upd = [&](int z, Upd &U) {  // z >= 0; plane n has z-faces only
+        const unsigned o = z * su, m = z < n ? su : 0, p = z * sw, k = z <= n ? sw : 0;
+        const auto ub = plane(a.b[0], o, m), uc = plane(a.c[0], o, m), vb = plane(a.b[1], o, m),
+                   vc = plane(a.c[1], o, m), wb = plane(a.b[2], p, k), wc = plane(a.c[2], p, k);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            U.ub[q] = ld(ub, fu[q]);
+            U.uc[q] = ld(uc, fu[q]);
+            U.vb[q] = ld(vb, fv[q]);
+            U.vc[q] = ld(vc, fv[q]);
+            U.wb[q] = ld(wb, fw[q]);
+            U.wc[q] = ld(wc, fw[q]);
+        }
+    };
+    // the norm's sums, per thread in LDS: in registers they would spill inside the march, where
+    // a reload waits for every load in flight
+    __shared__ double shS[3][64 * kS3W];
+    if (LAST)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) shS[d][threadIdx.x] = 0.0;
+    // one face at position q along d: R from T on its two sides (wall faces: 0, or in the explicit form half
+    // of the inner T); e = C - (1.5/dt) u*
+    auto face = [&](int d, int q, double tl, double tr, double base, double e) {
+        const bool end = q == 0 || q == n;
+        double R = 0.5 * (tl + tr);
+        if (end && !g.per[d]) R = g.pseudo ? 0.0 : 0.5 * (q == 0 ? tr : tl);
+        const double unew = base + a.rk * (R + e);
+        return unew;
+    };
+    auto norm = [&](int q, bool on, double base, double unew) {
+        const double df = on ? base - unew : 0.0;
+        return ((q == 0 || q == n) ? 0.5 : 1.0) * df * df;
+    };
+    // cell velocities of planes z .. z + 2, and of plane z its second difference and lower flux along z;
+    // z-faces z .. z + 2; the march starts at T of plane z0 - 1
+    double X0[2][3], X1[2][3], X2[2][3], dz[2][3], fz[2][3], w0[2], w1[2], w2[2];
+    Plane pn;  // plane z + 2 (z-faces z + 3), loaded at plane z - 1
+    {
+        Plane pa, pb, p0, p1;
+        double wa[2], xa[2][3], xb[2][3];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) wa[q] = ld(plane(a.s[2], face_of(z0 - 3, pz) * sw, sw), oc[q]);
+        load(z0 - 3, pa);
+        load(z0 - 2, pb);
+        load(z0 - 1, p0);
+        load(z0, p1);
+        load(z0 + 1, pn);
+        cells(z0 - 3, pa, wa, xa);
+        cells(z0 - 2, pb, pa.w, xb);
+        cells(z0 - 1, p0, pb.w, X0);
+        cells(z0, p1, p0.w, X1);
+        keep(z0 - 1, p0);
+        keep(z0, p1);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            w0[q] = pb.w[q];
+            w1[q] = p0.w[q];
+            w2[q] = p1.w[q];
+            const FaceVel f = face_vel(w0[q], a.kq[2]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                dz[q][c] = (xb[q][c] - 2.0 * X0[q][c]) + X1[q][c];
+                fz[q][c] = face_flux(f, xb[q][c], X0[q][c], (xa[q][c] - 2.0 * xb[q][c]) + X0[q][c], dz[q][c]);
+            }
+        }
+    }
+    Upd nxt{};                                      // of plane z at its top
+    double tv[2] = {0.0, 0.0}, tw[2] = {0.0, 0.0};  // plane z - 1: T_v, T_w
+    double vbl = 0.0, vel = 0.0;                    // and its lower row's v-face: base and e
+    double ru[2], rv[2], rw[2];                     // results to store
+    // the results formed at plane z (the lower row's v-faces are plane z - 1's)
+    auto flush = [&](int z) {
+        const unsigned o = z * su, m = z < n ? su : 0;
+        const auto u = plane(a.o[0], o, m), v = plane(a.o[1], o, m), vl = plane(a.o[1], o - su, z > z0 ? su : 0),
+                   w = plane(a.o[2], z * sw, sw);
+        st(vl, fv[0], rv[0]);
+        st(v, fv[1], rv[1]);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            st(u, fu[q], ru[q]);
+            st(w, fw[q], rw[q]);
+        }
+    };
+    for (int z = z0 - 1; z < z1; ++z) {
+        const int bf = z & 1;
+        cells(z + 2, pn, w2, X2);
+        keep(z + 2, pn);
+        const double w3[2] = {pn.w[0], pn.w[1]};
+        const Upd cur = nxt;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) shX[bf][c][2 * r + q][lane] = X0[q][c];
+        shT[bf][r][lane] = tv[1];
+        load(z + 3, pn);
+        load_upd(z + 1, nxt);
+        if (z > z0) flush(z - 1);
+        __syncthreads();
+        if (rowT) {
+            const double pu[2] = {shF[z & 3][0][2 * r][lane], shF[z & 3][0][2 * r + 1][lane]};
+            const double pv[3] = {shF[z & 3][1][2 * r][lane], shF[z & 3][1][2 * r + 1][lane], shF[z & 3][1][2 * r + 2][lane]};
+            double T[2][3];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                {   // z: the flux of the upper face
+                    const FaceVel f = face_vel(w1[q], a.kq[2]);
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const double D = (X0[q][c] - 2.0 * X1[q][c]) + X2[q][c];
+                        const double F = face_flux(f, X0[q][c], X1[q][c], dz[q][c], D);
+                        T[q][c] = (fz[q][c] - F) + a.kv[2] * dz[q][c];
+                        fz[q][c] = F;
+                        dz[q][c] = D;
+                    }
+                }
+                {   // x: the east face's flux is the next lane's
+                    const FaceVel f = face_vel(pu[q], a.kq[0]);
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const double X = X0[q][c], xm = lane_prev(X);
+                        const double D = (xm - 2.0 * X) + lane_next(X);
+                        const double F = face_flux(f, xm, X, lane_prev(D), D);
+                        T[q][c] += (F - lane_next(F)) + a.kv[0] * D;
+                    }
+                }
+            }
+            {   // y: the faces below, between and above the two rows
+                const FaceVel fs = face_vel(pv[0], a.kq[1]), fm = face_vel(pv[1], a.kq[1]), fn = face_vel(pv[2], a.kq[1]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const double XA = X0[0][c], XB = X0[1][c];
+                    const double s1 = shX[bf][c][2 * r - 1][lane], s2 = shX[bf][c][2 * r - 2][lane];
+                    const double n1 = shX[bf][c][2 * r + 2][lane], n2 = shX[bf][c][2 * r + 3][lane];
+                    const double DA = (s1 - 2.0 * XA) + XB, DB = (XA - 2.0 * XB) + n1;
+                    const double Fs = face_flux(fs, s1, XA, (s2 - 2.0 * s1) + XA, DA);
+                    const double Fm = face_flux(fm, XA, XB, DA, DB);
+                    const double Fn = face_flux(fn, XB, n1, DB, (XB - 2.0 * n1) + n2);
+                    T[0][c] += (Fs - Fm) + a.kv[1] * DA;
+                    T[1][c] += (Fm - Fn) + a.kv[1] * DB;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                ru[q] = face(0, i, lane_prev(T[q][0]), T[q][0], cur.ub[q], cur.uc[q] - g.c15 * pu[q]);
+                rw[q] = face(2, z, tw[q], T[q][2], cur.wb[q], cur.wc[q] - g.c15 * w0[q]);
+            }
+            rv[0] = face(1, y, shT[bf][r - 1][lane], tv[0], vbl, vel);
+            rv[1] = face(1, y + 1, T[0][1], T[1][1], cur.vb[1], cur.vc[1] - g.c15 * pv[1]);
+            if (LAST && z >= z0) {
+                shS[0][threadIdx.x] += norm(i, fu[0] != kNone && z < n, cur.ub[0], ru[0]) +
+                                       norm(i, fu[1] != kNone && z < n, cur.ub[1], ru[1]);
+                shS[1][threadIdx.x] += norm(y, fv[0] != kNone && z > z0, vbl, rv[0]) +
+                                       norm(y + 1, fv[1] != kNone && z < n, cur.vb[1], rv[1]);
+                shS[2][threadIdx.x] += norm(z, fw[0] != kNone, cur.wb[0], rw[0]) +
+                                       norm(z, fw[1] != kNone, cur.wb[1], rw[1]);
+            }
+            vbl = cur.vb[0];
+            vel = cur.vc[0] - g.c15 * pv[0];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                tv[q] = T[q][1];
+                tw[q] = T[q][2];
+            }
         }
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            w[c][0] = w[c][1]; w[c][1] = w[c][2]; w[c][2] = w[c][3]; w[c][3] = w[c][4]; w[c][4] = nw[c];
+        for (int q = 0; q < 2; ++q) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                X0[q][c] = X1[q][c];
+                X1[q][c] = X2[q][c];
+            }
+            w0[q] = w1[q];
+            w1[q] = w2[q];
+            w2[q] = w3[q];
         }
-        fzl = fzh;
-        fzh = nfz;
-        xc += sz;
+    }
+    flush(z1 - 1);
+    if (z1 <= n) {  // the lower rows' v-faces of the last plane
+        shT[z1 & 1][r][lane] = tv[1];
+        __syncthreads();
+        if (rowT) {
+            rv[0] = face(1, y, shT[z1 & 1][r - 1][lane], tv[0], vbl, vel);
+            if (LAST) shS[1][threadIdx.x] += norm(y, fv[0] != kNone, vbl, rv[0]);
+            st(plane(a.o[1], (unsigned)(z1 - 1) * su, su), fv[0], rv[0]);
+        }
+    }
+    if (LAST) {
+        double sq[3] = {shS[0][threadIdx.x], shS[1][threadIdx.x], shS[2][threadIdx.x]};
+        __syncthreads();
+        block_reduce_n<0u>(sq, &shX[0][0][0][0]);
+        if (threadIdx.x == 0)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) a.partials[3 * (int64_t)blk + d] = sq[d];
     }
 }
 
@@ -301,30 +619,29 @@ __global__ __launch_bounds__(B) void k_gen_update(Geom g, FaceArrays a, const do
     }
     if (last) {
         const double r = block_reduce<false>(sq, sh);
-        if (threadIdx.x == 0) partials[blk] = r;
+        if (threadIdx.x == 0)
+            for (int k = 0; k < 3; ++k) partials[3 * blk + k] = k == d ? r : 0.0;
     }
 }
 
-// Error_Computation from the per-direction block partials; the loop control
-// of main.cpp:898-1039 (countIter, IterNum cap, divergence guard), or for
-// PSEUDO_TIMESTEPPING = 0 the single update's norm with countIter 0
-__global__ __launch_bounds__(B) void k_gen_fin_pseudo(Geom g, const double *partials, int nb0, int nb1, int nb2,
-                                                      Ctl *ctl)
+// Error_Computation from the block partials (records of three, one sum per
+// direction); the loop control of main.cpp:898-1039 (countIter, IterNum cap,
+// divergence guard), or for PSEUDO_TIMESTEPPING = 0 the single update's norm
+// with countIter 0
+__global__ __launch_bounds__(1024) void k_gen_fin_pseudo(Geom g, const double *partials, int nrec, Ctl *ctl)
 {
-    __shared__ double sh[B / 64];
+    __shared__ double sh[48];
     if (ctl->mom_done) return;
-    const int nb[3] = {nb0, nb1, nb2};
-    double e[3] = {0.0, 0.0, 0.0};
-    int off = 0;
-    const double npts = (double)g.ncell;
-    for (int d = 0; d < g.dim; ++d) {
-        double s = 0.0;
-        for (int k = threadIdx.x; k < nb[d]; k += B) s += partials[off + k];
-        s = block_reduce<false>(s, sh);
-        if (threadIdx.x == 0) e[d] = sqrt(s) / sqrt(npts);
-        off += nb[d];
-    }
+    double v[3] = {0.0, 0.0, 0.0}, e[3] = {0.0, 0.0, 0.0};
+    for_records<3, 3>(partials, nrec, [&](const double *a) {
+        v[0] += a[0];
+        v[1] += a[1];
+        v[2] += a[2];
+    });
+    block_reduce_n<0u>(v, sh);
     if (threadIdx.x != 0) return;
+    const double npts = (double)g.ncell;
+    for (int d = 0; d < g.dim; ++d) e[d] = sqrt(v[d]) / sqrt(npts);
     double ne = (e[0] < e[1]) ? e[1] : e[0];
     if (g.dim == 3) ne = (ne < e[2]) ? e[2] : ne;
     ctl->norm_error = ne;
@@ -342,7 +659,7 @@ __global__ __launch_bounds__(B) void k_gen_fin_pseudo(Geom g, const double *part
 // ------------------------------------------------------------ BDF2 constant
 // main.cpp:879-884 with the pressure term folded: C = (1.5/dt) u^n + (0.5/dt)
 // (u^n - u^{n-1}) - G p (p's ghosts: Neumann mirror, so G p = 0 on wall
-// faces; periodic images); then u^{n-1} <- u^n and u^k = u* = u^n.
+// faces; periodic images); in 2D then u^{n-1} <- u^n and u^k = u* = u^n.
 struct Bdf2Arrays {
     double *u[3], *up[3], *c[3], *b[3], *s[3];
     const double *p;
@@ -368,6 +685,7 @@ __global__ __launch_bounds__(B) void k_gen_bdf2(Geom g, Bdf2Arrays a)
     }
     const double un = a.u[d][q], um = a.up[d][q];
     a.c[d][q] = g.c15 * un + (0.5 / g.dt) * (un - um) - gp;
+    if (!a.b[d]) return;  // 3D: the stages read u^n in place and the arrays change roles instead
     a.up[d][q] = un;
     a.b[d][q] = un;
     a.s[d][q] = un;
@@ -761,15 +1079,63 @@ hipError_t cells(const Ctx &c, hipStream_t s, double *const *f, double *X, const
 
 hipError_t flux(const Ctx &c, hipStream_t s, double *const *f, const double *X, double *T, const Ctl *guard)
 {
-    if (c.g.dim == 3 && c.flux_z) {
-        const int n = c.g.n, ntx = (n + kFzTX - 1) / kFzTX, nty = (n + kFzTY - 1) / kFzTY;
-        const int zc = c.flux_zc, nz = (n + zc - 1) / zc;
-        hipLaunchKernelGGL(k_gen_flux_z, dim3(ntx * nty * nz), dim3(256), 0, s, c.g, f[0], f[1], f[2], X, T, guard,
-                           ntx, nty, zc);
-        return hipGetLastError();
-    }
     hipLaunchKernelGGL(k_gen_flux, dim3(nblk(c.g.ncell)), dim3(B), 0, s, c.g, f[0], f[1],
                        c.g.dim == 3 ? f[2] : f[0], X, T, guard);
+    return hipGetLastError();
+}
+
+void stage3_shape(int n, int *ntx, int *nty, int *zc)
+{
+    *ntx = (n + 1 + kS3X - 1) / kS3X;
+    *nty = (n + 1 + kS3Y - 1) / kS3Y;
+    // one workgroup per CU: the chunk of planes for which the rounds of 256
+    // workgroups, each of zc planes and about five planes of prologue, are
+    // shortest
+    int64_t best = -1;
+    *zc = n + 1;
+    for (int q = 1; q <= n + 1; ++q) {
+        const int64_t blocks = (int64_t)*ntx * *nty * ((n + 1 + q - 1) / q);
+        const int64_t cost = (blocks + 255) / 256 * (q + 5);
+        if (best < 0 || cost <= best) { best = cost; *zc = q; }
+    }
+}
+
+int stage3_blocks(const Ctx &c)
+{
+    return c.s3_ntx * c.s3_nty * ((c.g.n + 1 + c.s3_zc - 1) / c.s3_zc);
+}
+
+hipError_t stage3(const Ctx &c, hipStream_t s, double *const *in, double *const *base, double *const *out, double rk,
+                  int last, const Ctl *guard)
+{
+    Stage3 a{};
+    for (int d = 0; d < 3; ++d) {
+        if (out[d] == in[d] || out[d] == base[d]) return hipErrorInvalidValue;
+        a.s[d] = in[d];
+        a.b[d] = base[d];
+        a.c[d] = c.C[d];
+        a.o[d] = out[d];
+    }
+    a.partials = c.partials;
+    a.rk = rk;
+    for (int d = 0; d < 3; ++d) {
+        a.kq[d] = -0.125 * c.g.idx[d];
+        a.kv[d] = c.g.idx2[d] * c.g.iren;
+        for (int hi = 0; hi < 2; ++hi) {
+            // 0: -mirror, 1: slip, 2: 2 - mirror, 3: 2 inflow - mirror
+            const int kind = hi ? c.g.kind_hi[d] : c.g.kind_lo[d];
+            for (int q = 0; q < 3; ++q) {
+                a.sg[2 * d + hi][q] = kind == 1 && q != d ? 1.0 : -1.0;
+                a.ct[2 * d + hi][q] = kind == 2 ? 2.0 : (kind == 3 ? 2.0 * c.g.inflow[q] : 0.0);
+            }
+        }
+    }
+    a.ntx = c.s3_ntx;
+    a.nty = c.s3_nty;
+    a.zc = c.s3_zc;
+    const dim3 grid(stage3_blocks(c));
+    if (last) hipLaunchKernelGGL(k_gen_stage3<true>, grid, dim3(64 * kS3W), 0, s, c.g, a, guard);
+    else hipLaunchKernelGGL(k_gen_stage3<false>, grid, dim3(64 * kS3W), 0, s, c.g, a, guard);
     return hipGetLastError();
 }
 
@@ -789,8 +1155,8 @@ hipError_t update(const Ctx &c, hipStream_t s, double rk, int last, const Ctl *g
 
 hipError_t fin_pseudo(const Ctx &c, hipStream_t s, Ctl *ctl)
 {
-    hipLaunchKernelGGL(k_gen_fin_pseudo, dim3(1), dim3(B), 0, s, c.g, c.partials, c.nb_face[0], c.nb_face[1],
-                       c.g.dim == 3 ? c.nb_face[2] : 0, ctl);
+    const int nrec = c.g.dim == 3 ? stage3_blocks(c) : c.nb_face[0] + c.nb_face[1];
+    hipLaunchKernelGGL(k_gen_fin_pseudo, dim3(1), dim3(1024), 0, s, c.g, c.partials, nrec, ctl);
     return hipGetLastError();
 }
 
@@ -802,8 +1168,8 @@ hipError_t bdf2(const Ctx &c, hipStream_t s)
         a.u[d] = on ? c.U[d] : nullptr;
         a.up[d] = on ? c.Up[d] : nullptr;
         a.c[d] = on ? c.C[d] : nullptr;
-        a.b[d] = on ? c.B[d] : nullptr;
-        a.s[d] = on ? c.S[d] : nullptr;
+        a.b[d] = on && c.g.dim == 2 ? c.B[d] : nullptr;
+        a.s[d] = on && c.g.dim == 2 ? c.S[d] : nullptr;
         a.nb[d] = on ? c.nb_face[d] : 0;
     }
     a.p = c.p;

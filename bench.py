@@ -221,7 +221,7 @@ def amr_leg(api, W, n0, steps, torch):
 def general_leg(api, n, steps, torch):
     """The general path on a 3D lid-driven cavity: n^3 cells, walls 135 with the
     lid (165, u = 1) on the y-hi side, Re = 1000, FP64, from rest after two
-    warm-up steps; plus the three per-stage kernels' rates."""
+    warm-up steps; plus the rates of the cell-velocity pass and of the stage kernel."""
     import numpy as np
     inp = api.default_inputs(n_cell=n, max_grid_size=(n, n, n), IterNum=100, cfl=0.5, ren=1000.0, vis=1e-3,
                              phy_bc_lo=(135, 135, 135), phy_bc_hi=(135, 165, 135), inflow_waveform=(1.0, 0.0, 0.0),
@@ -235,8 +235,8 @@ def general_leg(api, n, steps, torch):
     torch.cuda.synchronize()
     sec = time.perf_counter() - t0
     names = {7: "amr::gen::k_gen_cells (cell velocities with ghosts)",
-             8: "amr::gen::k_gen_flux (QUICK + viscous fluxTotal)",
-             9: "amr::gen::k_gen_update (stage update of every face)"}
+             8: "amr::gen::k_gen_stage3 (one RK4 stage)",
+             9: "amr::gen::k_gen_stage3 (one RK4 stage + norm partials)"}
     kern = []
     for which, name in names.items():
         ms, nbytes = ctx.time_kernel(which, reps=10)

@@ -146,6 +146,18 @@ def test_3d_steps_match_oracle(bc_lo, bc_hi, init):
     _check(ref, ref_stats, got, stats, 3)
 
 
+@pytest.mark.parametrize("bc_lo,bc_hi", [((-135, 165, 135), (135, 165, -135)),   # slip, inflow and lid sides
+                                         ((111, 135, 111), (111, 165, 111)),     # periodic x and z
+                                         ((135, 111, 135), (1, 111, 165))])      # periodic y, east slip
+@pytest.mark.parametrize("n", [4, 5, 7, 10, 20, 32, 56, 64])
+def test_3d_stage_kernel_tile_edges(n, bc_lo, bc_hi):
+    """The one-pass 3D stage at the edges of its tiles (58 columns x 11 rows, chunks of planes): sizes below
+    one tile, whole tiles of rows (n + 1 = 11, 33), one row past (n + 1 = 5, 21), the last size of one
+    column tile (n + 1 = 57) and the first of two."""
+    ref, ref_stats, got, stats, _, _ = _run_pair(3, n, 150.0, bc_lo, bc_hi, 2, inflow=(0.4, 0.2, -0.3), amp=0.1)
+    _check(ref, ref_stats, got, stats, 3)
+
+
 @pytest.mark.parametrize("dim", [2, 3])
 def test_explicit_time_marching_matches_oracle(dim):
     bc_lo = (111, 135, 135)
