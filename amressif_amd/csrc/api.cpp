@@ -543,6 +543,18 @@ int launch_pseudo_iteration(amressif_ctx *ctx, int it, int *nb)
     amr::StageLaunch a{};
     a.ub = c.U[0]; a.vb = c.U[1]; a.cu = c.C[0]; a.cv = c.C[1]; a.p = c.p;
     a.foldp = 1;  // C holds -G p (amr_momentum_begin)
+    if (amr::iter_tile_wanted(c)) {
+        // u^k into S1, then S1 becomes u^k (a launch skipped after convergence copies u^k to S1)
+        a.uo = c.S1[0]; a.vo = c.S1[1];
+        // (it moves 48 B per cell: u^k, v^k, c_u, c_v in, u^{k+1}, v^{k+1} out; its record keeps the
+        // bytes of the two two-stage passes it counts as)
+        HIPCHK(amr::kprof_begin(c, amr::KP_ITER, amr::KL_MOM, it, 2 * 64.0 * (double)c.g.n * c.g.n));
+        HIPCHK(amr::launch_iteration(c, a, nb));
+        HIPCHK(amr::kprof_end(c));
+        std::swap(c.U[0], c.S1[0]);
+        std::swap(c.U[1], c.S1[1]);
+        return 0;
+    }
     if (c.stage_pair && amr::stage_pair_fits(c)) {
         // stages 1-2 from u^k into S2, stages 3-4 from S2 into S1, then S1 becomes
         // u^k (a launch skipped after convergence copies u^k to S1)
@@ -634,9 +646,12 @@ hipError_t kprof_collect(const Ctx &c)
             float ms = 0.f;
             hipError_t err = hipEventElapsedTime(&ms, r.e0, r.e1);
             if (err != hipSuccess) return err;
-            k->sum_ms[r.id] += ms;
-            k->sum_bytes[r.id] += r.bytes;
-            k->cnt[r.id] += 1;
+            const bool both = r.id == KP_ITER;
+            for (int id = both ? KP_PAIR : r.id; id <= (both ? KP_PAIR_LAST : r.id); ++id) {
+                k->sum_ms[id] += both ? 0.5 * ms : ms;
+                k->sum_bytes[id] += both ? 0.5 * r.bytes : r.bytes;
+                k->cnt[id] += 1;
+            }
         }
         k->pool.push_back(r.e0);
         k->pool.push_back(r.e1);
@@ -814,6 +829,9 @@ int amressif_create(const amressif_inputs *in, void *hip_stream, amressif_ctx **
     if (const char *e = std::getenv("AMRESSIF_STAGE_ORDER")) c.stage_order = std::atoi(e) ? 1 : 0;
     if (const char *e = std::getenv("AMRESSIF_STAGE_ALT")) c.stage_alt = std::atoi(e) ? 1 : 0;
     if (const char *e = std::getenv("AMRESSIF_STAGE_FAST")) c.stage_fast = std::atoi(e) ? 1 : 0;
+    // a named form of the two-stage launches is the form asked for
+    if (std::getenv("AMRESSIF_STAGE_PAIR") || std::getenv("AMRESSIF_PAIR_ROWS")) c.iter_tile = 0;
+    if (const char *e = std::getenv("AMRESSIF_ITER_TILE")) c.iter_tile = std::max(0, std::min(2, std::atoi(e)));
     if (const char *e = std::getenv("AMRESSIF_STAGE_PAIR")) c.stage_pair = std::atoi(e) ? 1 : 0;
     if (const char *e = std::getenv("AMRESSIF_PAIR_ROWS")) c.pair_rows = std::max(4, std::min(256, std::atoi(e)));
     if (const char *e = std::getenv("AMRESSIF_MIXED_PAIR")) c.mixed_pair = std::atoi(e) ? 1 : 0;
@@ -1781,8 +1799,8 @@ int amressif_time_kernel(amressif_ctx *ctx, int which, int reps, int64_t copy_by
         HIPCHK(hipMalloc(&src, (size_t)copy_bytes));
         HIPCHK(hipMalloc(&dst, (size_t)copy_bytes));
         HIPCHK(hipMemsetAsync(src, 0, (size_t)copy_bytes, c.stream));
-    } else if (which < 0 || (which > 6 && which != 10)) {
-        return fail(ctx, AMRESSIF_ERR_ARG, "which must be 0..6 or 10");
+    } else if (which < 0 || (which > 6 && which != 10 && which != 11)) {
+        return fail(ctx, AMRESSIF_ERR_ARG, "which must be 0..6, 10 or 11");
     }
     if (which == 6 && !amr::stage_pair_fits(c)) return fail(ctx, AMRESSIF_ERR_ARG, "no two-stage kernel at this size");
     if ((which == 3 || which == 4 || which == 10) && c.in.precision != AMRESSIF_MIXED)
@@ -1836,6 +1854,14 @@ int amressif_time_kernel(amressif_ctx *ctx, int which, int reps, int64_t copy_by
             int nb = 0;
             return amr::launch_stage_pair(c, a, &nb);
         }
+        if (which == 11) {  // a whole pseudo-iteration, u^k from U into S2
+            amr::StageLaunch a{};
+            a.ub = c.U[0]; a.vb = c.U[1]; a.cu = c.C[0]; a.cv = c.C[1];
+            a.uo = c.S2[0]; a.vo = c.S2[1];
+            a.unguarded = 1;
+            int nb = 0;
+            return amr::launch_iteration(c, a, &nb);
+        }
         if (which == 1 || which == 5) return amr::launch_smooth_fine(c, which, c.S2[0]);
         return amr::launch_copy_bytes(c, src, dst, copy_bytes);
     };
@@ -1866,10 +1892,10 @@ int amressif_time_kernel(amressif_ctx *ctx, int which, int reps, int64_t copy_by
         // 5 finest up-leg smoother + FP64 outer step: reads e, r (2 t), the coarse e (t / 4),
         //   phi, b (2 x 8 B), writes phi (8 B) and the next r (t);
         // 6 two FP64 stages in one pass: the stage's 64 B (the first stage stays in registers);
-        // 10 mixed iteration in one pass: reads u^k, v^k, c_u, c_v, writes u^{k+1}, v^{k+1} (6 x 8 B)
+        // 10, 11 mixed iteration, FP64 pseudo-iteration in one pass: reads u^k, v^k, c_u, c_v, writes u^{k+1}, v^{k+1} (6 x 8 B)
         const double t = c.in.precision == AMRESSIF_MIXED ? 4.0 : 8.0;
         const double per_cell[7] = {64.0, 2.25 * t, 0.0, 48.0, 48.0, 3.25 * t + 24.0, 64.0};
-        *bytes_per_launch = which == 2 ? 2.0 * (double)copy_bytes : which == 10 ? 48.0 * cells : per_cell[which] * cells;
+        *bytes_per_launch = which == 2 ? 2.0 * (double)copy_bytes : which >= 10 ? 48.0 * cells : per_cell[which] * cells;
     }
     return AMRESSIF_OK;
 }

@@ -5,7 +5,7 @@
 //
 // Layout in HBM (one box, i fastest, then j, then k; no padding):
 //   face array of direction d: n + 1 along d, n along the others
-//   cell arrays (p, phi, b, multigrid levels, fluxTotal comps): n^dim
+//   cell arrays (p, phi, b, multigrid levels): n^dim
 //   cell velocities X: dim comps with two ghost layers, (n + 4)^dim each
 //   (in 2D the k extent is 1 and has no ghosts)
 #pragma once
@@ -51,9 +51,8 @@ struct Level {
 struct Ctx {
     Geom g{};
     double rk[4]{};
-    double *U[3]{}, *Up[3]{}, *C[3]{}, *B[3]{}, *S[3]{};  // u^n, u^{n-1}, BDF2 constant, pseudo base, u*
+    double *U[3]{}, *Up[3]{}, *C[3]{}, *B[3]{}, *S[3]{};  // u^n, u^{n-1}, BDF2 constant, pseudo bases (u* ends in S)
     double *X = nullptr;   // cell velocities with ghosts
-    double *T = nullptr;   // fluxTotal (dim comps, n^dim)
     double *p = nullptr, *phi = nullptr, *b = nullptr;
     Level lev[kMaxGenLevels]{};
     int nlev = 0;
@@ -61,7 +60,7 @@ struct Ctx {
     int mb = 0;
     double *partials = nullptr;
     int64_t npartials = 0;
-    int nb_face[3]{};        // blocks per face direction in k_gen_update
+    int nb_face[3]{};        // blocks per face direction of a launch over every face
     int last_P = 8, last_V = 8;
     int s3_ntx = 0, s3_nty = 0, s3_zc = 0;  // 3D stage: tiles in x and y, planes per workgroup
 };
@@ -69,10 +68,8 @@ struct Ctx {
 // ---- launchers (kernels_gen.hip); every guarded kernel returns at once once
 // its loop's flag in the control block is set
 hipError_t cells(const Ctx &c, hipStream_t s, double *const *faces, double *X, const Ctl *guard);
-hipError_t flux(const Ctx &c, hipStream_t s, double *const *faces, const double *X, double *T, const Ctl *guard);
-// stage update of every face: u* <- u^k + rk (R - c15 u* + C); last: the
-// norm partials of u^k - u* and u^k <- u* as well
-hipError_t update(const Ctx &c, hipStream_t s, double rk, int last, const Ctl *guard);
+// 2D: one pseudo-iteration (or the explicit update), out <- the last stage from base; with its norm partials
+hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, const Ctl *guard);
 // 3D: one RK4 stage in one pass, out <- base + rk (R(in) - c15 in + C); out
 // aliases neither in nor base.  last: the norm partials of base - out as well
 hipError_t stage3(const Ctx &c, hipStream_t s, double *const *in, double *const *base, double *const *out, double rk,

@@ -18,6 +18,7 @@
 #include <cstdlib>
 
 #include "gen.hpp"
+#include "iter_tile.hpp"
 
 namespace {
 
@@ -263,15 +264,13 @@ int amr_gen_create(amressif_ctx *ctx)
         GALLOC(&gc.B[d], g.nf[d]); GALLOC(&gc.S[d], g.nf[d]);
     }
     GALLOC(&gc.X, (size_t)g.xs * dim);
-    if (dim == 2) GALLOC(&gc.T, cellsz * dim);
     GALLOC(&gc.p, cellsz); GALLOC(&gc.phi, cellsz); GALLOC(&gc.b, cellsz);
     for (int l = 0; l < gc.nlev; ++l) {
         GALLOC(&gc.lev[l].e, (size_t)gc.lev[l].ncell);
         GALLOC(&gc.lev[l].r, (size_t)gc.lev[l].ncell);
     }
     gc.npartials = std::max<int64_t>(2 * ((g.ncell + G::kBlock - 1) / G::kBlock),
-                                     3 * (dim == 3 ? (int64_t)G::stage3_blocks(gc)
-                                                   : (int64_t)gc.nb_face[0] + gc.nb_face[1])) + 64;
+                                     3 * (int64_t)(dim == 3 ? G::stage3_blocks(gc) : amr::iter_tile_blocks(n))) + 64;
     GALLOC(&gc.partials, (size_t)gc.npartials);
     {
         std::vector<double> pinv;
@@ -552,64 +551,44 @@ int amr_gen_advance(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats)
     for (int s = 0; s < nsteps; ++s) {
         GCHK(G::bdf2(gc, c.stream));
         GCHK(amr::launch_ctl_reset_step(c));
-        // ---- momentum predictor
-        if (dim3) {
-            // u^{n-1}'s array is free once the constant holds it, and becomes the
-            // scratch of stages 1 and 3; stages 2 and 4 of pseudo-iteration k write
-            // the array (k odd: B, even: S) that then is the base of the next one
-            double **F[3] = {gc.Up, gc.B, gc.S};
-            auto iter_out = [&](int k) { return F[(k & 1) ? 1 : 2]; };
-            int count;
-            if (!g.pseudo) {
-                GCHK(G::stage3(gc, c.stream, gc.U, gc.U, iter_out(1), g.dt / 1.5, 1, c.ctl));
-                GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
-                count = 1;
-            } else {
-                int done = 0, batch = std::max(1, gc.last_P), k = 0;
-                while (!done) {
-                    for (int it = 0; it < batch; ++it) {
-                        double **base = k == 0 ? gc.U : iter_out(k), **out = iter_out(k + 1);
-                        GCHK(G::stage3(gc, c.stream, base, base, F[0], gc.rk[0], 0, c.ctl));
-                        GCHK(G::stage3(gc, c.stream, F[0], base, out, gc.rk[1], 0, c.ctl));
-                        GCHK(G::stage3(gc, c.stream, out, base, F[0], gc.rk[2], 0, c.ctl));
-                        GCHK(G::stage3(gc, c.stream, F[0], base, out, gc.rk[3], 1, c.ctl));
-                        GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
-                        ++k;
-                    }
-                    if (int rc = poll(ctx)) return rc;
-                    done = c.ctl_host->mom_done;
-                    batch = std::max(2, batch / 2);
-                }
-                count = std::max(1, c.ctl_host->mom_count);  // launches past it left every array as it was
-                gc.last_P = count;
-            }
-            // u* is iter_out(count)'s; u^n becomes u^{n-1}, and the projection
-            // writes u^{n+1} into the scratch
-            for (int d = 0; d < 3; ++d) {
-                if (count & 1) std::swap(gc.B[d], gc.S[d]);
-                std::swap(gc.U[d], gc.Up[d]);
-            }
-        } else if (!g.pseudo) {
-            GCHK(G::cells(gc, c.stream, gc.S, gc.X, c.ctl));
-            GCHK(G::flux(gc, c.stream, gc.S, gc.X, gc.T, c.ctl));
-            GCHK(G::update(gc, c.stream, g.dt / 1.5, 1, c.ctl));
+        // ---- momentum predictor: pseudo-iteration k writes the array (k odd: B, even: S)
+        // that is the base of the next one.  u^{n-1}'s array is free once the constant
+        // holds it: the scratch of the 3D stages 1 and 3
+        double **scratch = gc.Up;
+        auto iter_out = [&](int k) { return (k & 1) ? gc.B : gc.S; };
+        int count = 1;
+        if (!g.pseudo) {
+            if (dim3) GCHK(G::stage3(gc, c.stream, gc.U, gc.U, iter_out(1), g.dt / 1.5, 1, c.ctl));
+            else GCHK(G::iteration2(gc, c.stream, gc.U, iter_out(1), c.ctl));
             GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
         } else {
-            int done = 0, batch = std::max(1, gc.last_P);
+            int done = 0, batch = std::max(1, gc.last_P), k = 0;
             while (!done) {
                 for (int it = 0; it < batch; ++it) {
-                    for (int sub = 0; sub < 4; ++sub) {
-                        GCHK(G::cells(gc, c.stream, gc.S, gc.X, c.ctl));
-                        GCHK(G::flux(gc, c.stream, gc.S, gc.X, gc.T, c.ctl));
-                        GCHK(G::update(gc, c.stream, gc.rk[sub], sub == 3, c.ctl));
+                    double **base = k == 0 ? gc.U : iter_out(k), **out = iter_out(k + 1);
+                    if (dim3) {
+                        GCHK(G::stage3(gc, c.stream, base, base, scratch, gc.rk[0], 0, c.ctl));
+                        GCHK(G::stage3(gc, c.stream, scratch, base, out, gc.rk[1], 0, c.ctl));
+                        GCHK(G::stage3(gc, c.stream, out, base, scratch, gc.rk[2], 0, c.ctl));
+                        GCHK(G::stage3(gc, c.stream, scratch, base, out, gc.rk[3], 1, c.ctl));
+                    } else {
+                        GCHK(G::iteration2(gc, c.stream, base, out, c.ctl));
                     }
                     GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
+                    ++k;
                 }
                 if (int rc = poll(ctx)) return rc;
                 done = c.ctl_host->mom_done;
                 batch = std::max(2, batch / 2);
             }
-            gc.last_P = std::max(1, c.ctl_host->mom_count);
+            count = std::max(1, c.ctl_host->mom_count);  // launches past it left every array as it was
+            gc.last_P = count;
+        }
+        // u* is iter_out(count)'s; u^n becomes u^{n-1}, and the projection writes
+        // u^{n+1} into the scratch
+        for (int d = 0; d < g.dim; ++d) {
+            if (count & 1) std::swap(gc.B[d], gc.S[d]);
+            std::swap(gc.U[d], gc.Up[d]);
         }
         // ---- Poisson: b = (1.5/dt) D(u*), its mean removed in the residual
         int nb = 0;
@@ -652,8 +631,7 @@ int amr_gen_advance(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats)
 }
 
 // ================================================================== timing
-// which: 0 cells; 1, 2: 2D the fluxTotal and update passes of a stage, 3D the
-// whole stage without and with the norm partials
+// which: 0 cells; 1: 3D one stage, 2: with the norm partials; 2D 1 and 2: one pseudo-iteration
 int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, double *bytes_per_launch)
 {
     Ctx &c = ctx->c;
@@ -663,21 +641,14 @@ int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, 
     hipEvent_t e0, e1;
     GCHK(hipEventCreate(&e0));
     GCHK(hipEventCreate(&e1));
-    // a realistic state: S = U, X and T of it
-    for (int d = 0; d < g.dim; ++d) {
-        GCHK(hipMemcpyAsync(gc.S[d], gc.U[d], g.nf[d] * 8, hipMemcpyDeviceToDevice, c.stream));
+    // a realistic state: the pseudo base another array than the stencil input
+    for (int d = 0; d < g.dim; ++d)
         GCHK(hipMemcpyAsync(gc.B[d], gc.U[d], g.nf[d] * 8, hipMemcpyDeviceToDevice, c.stream));
-    }
     GCHK(G::bdf2(gc, c.stream));
-    if (g.dim == 2) {
-        GCHK(G::cells(gc, c.stream, gc.S, gc.X, nullptr));
-        GCHK(G::flux(gc, c.stream, gc.S, gc.X, gc.T, nullptr));
-    }
     auto launch = [&]() -> hipError_t {
         if (which == 0) return G::cells(gc, c.stream, gc.U, gc.X, nullptr);
         if (g.dim == 3) return G::stage3(gc, c.stream, gc.U, gc.B, gc.S, gc.rk[0], which == 2, nullptr);
-        if (which == 1) return G::flux(gc, c.stream, gc.S, gc.X, gc.T, nullptr);
-        return G::update(gc, c.stream, 0.0, 0, nullptr);  // rk = 0: the faces keep their values
+        return G::iteration2(gc, c.stream, gc.B, gc.S, nullptr);
     };
     GCHK(launch());
     GCHK(hipEventRecord(e0, c.stream));
@@ -690,16 +661,10 @@ int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, 
     (void)hipEventDestroy(e1);
     *avg_ms = ms / reps;
     // algorithmic bytes (FP64), each array read or written once per launch:
-    // cells: dim face arrays in, dim ghosted cell comps out; flux: dim face
-    // arrays and X in, T out; update: T, u*, u^k, C in, u* out; the 3D stage:
-    // u*, u^k, C in, u* out
+    // cells: dim face arrays in, dim ghosted cell comps out; the 3D stage: u*,
+    // u^k, C in, u* out; the 2D pseudo-iteration: u^k, C in, u^{k+1} out
     const double faces = (double)(g.nf[0] + g.nf[1] + (g.dim == 3 ? g.nf[2] : 0));
-    const double cellsd = (double)g.ncell * g.dim;
-    double bytes = 0.0;
-    if (which == 0) bytes = 8.0 * (faces + (double)g.xs * g.dim);
-    else if (g.dim == 3) bytes = 8.0 * 4.0 * faces;
-    else if (which == 1) bytes = 8.0 * (faces + (double)g.xs * g.dim + cellsd);
-    else bytes = 8.0 * (cellsd + 4.0 * faces);
+    const double bytes = which == 0 ? 8.0 * (faces + (double)g.xs * g.dim) : 8.0 * (g.dim == 3 ? 4.0 : 3.0) * faces;
     if (bytes_per_launch) *bytes_per_launch = bytes;
     c.pred_valid = 0;
     return AMRESSIF_OK;

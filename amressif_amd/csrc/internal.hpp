@@ -104,7 +104,8 @@ enum KProfId {
     KP_PAIR,         // k_stage_pair<false>: FP64 RK stages 1-2
     KP_PAIR_LAST,    // k_stage_pair<true>: FP64 RK stages 3-4 + norm partials
     KP_MPAIR,        // k_mixed_pair: mixed residual + tangent-linear update in one pass
-    KP_COUNT
+    KP_COUNT,
+    KP_ITER = KP_COUNT  // k_iter_tile, all four stages: half its record to KP_PAIR, half to KP_PAIR_LAST
 };
 enum KProfLoop { KL_MOM = 0, KL_MG, KL_PHASE, KL_ONCE, KL_PROJ };
 struct KProf {
@@ -153,6 +154,7 @@ struct Ctx {
     int stage_fast = 1;      // k_stage64: unrolled interior path (0: every wave on the general march)
     int stage_pair = 1;      // FP64 pseudo-iteration as two k_stage_pair launches (0: four k_stage64)
     int pair_rows = 16;      // k_stage_pair: output rows per wave
+    int iter_tile = 1;       // FP64 pseudo-iteration as one k_iter_tile launch where its rule says so (0: never, 2: at every size)
     // mixed iteration as one k_mixed_pair launch (0: k_stage64 mode 3 + k_tangent);
     // used by the step without a tape (advance) with the multigrid solve
     int mixed_pair = 1;
@@ -248,6 +250,9 @@ hipError_t launch_stage(const Ctx &c, const StageLaunch &a, int *nblocks);
 // (+ norm partials).  uo must differ from us and ub.
 hipError_t launch_stage_pair(const Ctx &c, const StageLaunch &a, int *nblocks);
 bool stage_pair_fits(const Ctx &c);
+// one pseudo-iteration in one launch (k_iter_tile) from the base a.ub, a.vb into a.uo, a.vo
+bool iter_tile_wanted(const Ctx &c);
+hipError_t launch_iteration(const Ctx &c, const StageLaunch &a, int *nblocks);
 // cu, cv += -G p on the interior faces, once per FP64 step (p fixed over its pseudo-iterations)
 hipError_t launch_fold_gradp(const Ctx &c);
 // mixed (defect-correction) pseudo-iteration: see kernels_stage.hip

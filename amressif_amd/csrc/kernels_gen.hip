@@ -1,21 +1,16 @@
 // Kernels of the general path (gen.hpp): the fractional step on n^dim cells,
 // dim 2 or 3, with periodic directions beside the wall codes, FP64.
 //
-// One RK4 dual-time stage is one pass in 3D (k_gen_stage3) and three streaming
-// passes in 2D:
-//   k_gen_cells  : cell velocities X from the faces with every ghost layer the
-//                  stencils read (cont2cart, utilities.cpp:16-350; periodic
-//                  images and the wall rules, corners in the reference's pass
-//                  order);
-//   k_gen_flux   : fluxTotal T = -C + V per cell: the QUICK half-node fluxes
-//                  of both faces per direction (fn_flux_calc.cpp:11-202) and
-//                  the viscous Laplacian (:695-766), X read through L2;
-//   k_gen_update : every face: R = (T(left) + T(right))/2 with the flux ghosts
-//                  of main.cpp:939-1014 (wall faces R = 0, periodic images),
-//                  u* <- u^k + rk (R - (1.5/dt) u* + C), the BDF2 constant C
-//                  holding -G p (momentum.cpp:68-87, fn_rhs.cpp:8-68); on the
-//                  last stage the Error_Computation partials (utilities.cpp:
-//                  421-493) and u^k <- u*.
+// The RK4 dual-time loop (momentum.cpp:9-94): in 3D one launch per stage
+// (k_gen_stage3), in 2D one per pseudo-iteration of four stages (k_iter_tile,
+// kernels_iter.hip).  A stage forms cell velocities with the wall rules or
+// periodic images (cont2cart, utilities.cpp:16-350), fluxTotal T = -C + V per
+// cell (QUICK, fn_flux_calc.cpp:11-202, and the viscous Laplacian :695-766), and
+// on every face R = (T(left) + T(right))/2 with the flux ghosts of
+// main.cpp:939-1014 (wall faces R = 0, periodic images), u* <- u^k + rk (R -
+// (1.5/dt) u* + C), the BDF2 constant C holding -G p (momentum.cpp:68-87,
+// fn_rhs.cpp:8-68); on the last stage the Error_Computation partials
+// (utilities.cpp:421-493).  k_gen_cells writes the cell velocities for output.
 // Then the Poisson RHS (fn_rhs.cpp:71-125), a geometric V-cycle iteration with
 // red-black Gauss-Seidel on Neumann / periodic neighbours and a dense
 // pseudo-inverse bottom (poisson.cpp:41-186), and the projection
@@ -23,6 +18,7 @@
 // (xcd_block), so the rows and planes a stencil shares sit in one L2.
 #include "device_common.hpp"
 #include "gen.hpp"
+#include "iter_tile.hpp"
 
 namespace amr {
 namespace gen {
@@ -115,60 +111,6 @@ __global__ __launch_bounds__(B) void k_gen_cells(Geom g, const double *f0, const
 #pragma unroll
     for (int c = 0; c < 3; ++c)
         if (c < g.dim) X[q + (int64_t)c * g.xs] = v[c];
-}
-
-// ------------------------------------------------------------ fluxTotal
-__device__ __forceinline__ double quick(double vel, double a2, double a1, double b0, double b1)
-{
-    return quick_flux<double>(vel, a2, a1, b0, b1);
-}
-
-__global__ __launch_bounds__(B) void k_gen_flux(Geom g, const double *f0, const double *f1, const double *f2,
-                                                const double *X, double *T, const Ctl *guard)
-{
-    if (guard && guard->mom_done) return;
-    const int64_t q = gid();
-    if (q >= g.ncell) return;
-    const int n = g.n;
-    int x[3];
-    split3(q, n, n, x);
-    const double *f[3] = {f0, f1, f2};
-    const int64_t xc = xidx(g, x[0], x[1], x[2]);
-    int64_t st[3];
-    st[0] = 1;
-    st[1] = n + 4;
-    st[2] = (int64_t)(n + 4) * (n + 4);
-    // face velocities of both faces per direction
-    double fw[3], fe[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (d >= g.dim) break;
-        int e[3] = {x[0], x[1], x[2]};
-        e[d] += 1;
-        fw[d] = f[d][fidx(g, d, x[0], x[1], x[2])];
-        fe[d] = f[d][fidx(g, d, e[0], e[1], e[2])];
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        if (c >= g.dim) break;
-        const double *Xc = X + (int64_t)c * g.xs + xc;
-        double conv = 0.0, lap[3] = {0.0, 0.0, 0.0};
-        const double C = Xc[0];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            if (d >= g.dim) break;
-            const int64_t o = st[d];
-            const double m2 = Xc[-2 * o], m1 = Xc[-o], p1 = Xc[o], p2 = Xc[2 * o];
-            const double Fw = quick(fw[d], m2, m1, C, p1), Fe = quick(fe[d], m1, C, p1, p2);
-            const double t = (Fe - Fw) * g.idx[d];
-            conv = d == 0 ? t : conv + t;
-            lap[d] = (p1 - 2.0 * C + m1) * g.idx2[d];
-        }
-        // ((E - 2C + W)/dx^2 + (N - 2C + S)/dy^2)/ren [+ ((B - 2C + F)/dz^2)/ren]
-        double visc = (lap[0] + lap[1]) * g.iren;
-        if (g.dim == 3) visc = visc + lap[2] * g.iren;
-        T[q + (int64_t)c * g.ncell] = (0.0 - conv) + visc;
-    }
 }
 
 // A face's velocity as the three factors its QUICK fluxes share: with X(-), X(+) the
@@ -572,58 +514,6 @@ __device__ __forceinline__ void face_coords(const Geom &g, int d, int64_t q, int
     split3(q, g.n + (d == 0), g.n + (d == 1), x);
 }
 
-struct FaceArrays {
-    double *s[3], *b[3];
-    const double *c[3];
-    int nb[3];
-};
-
-// ------------------------------------------------------------ stage update
-__global__ __launch_bounds__(B) void k_gen_update(Geom g, FaceArrays a, const double *T, double rk, int last,
-                                                  double *partials, const Ctl *guard)
-{
-    __shared__ double sh[B / 64];
-    if (guard && guard->mom_done) return;
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
-    int lb;
-    const int d = face_dir(a.nb, blk, lb);
-    const int64_t q = (int64_t)lb * B + threadIdx.x;
-    const int n = g.n;
-    double sq = 0.0;
-    if (q < g.nf[d]) {
-        int x[3];
-        face_coords(g, d, q, x);
-        const int xd = x[d];
-        const bool wlo = xd == 0 && !g.per[d], whi = xd == n && !g.per[d];
-        double R;
-        if (g.pseudo && (wlo || whi)) {
-            R = 0.0;  // the wall ghost -T(mirror) cancels T (main.cpp:953-1012)
-        } else {
-            int l[3] = {x[0], x[1], x[2]}, r[3] = {x[0], x[1], x[2]};
-            l[d] = xd == 0 ? n - 1 : xd - 1;
-            r[d] = xd == n ? 0 : xd;
-            const double *Td = T + (int64_t)d * g.ncell;
-            // explicit form: fluxTotal's wall ghosts keep setVal's 0
-            const double tl = wlo ? 0.0 : Td[cidx(g, l)], tr = whi ? 0.0 : Td[cidx(g, r)];
-            R = 0.5 * (tl + tr);
-        }
-        const double us = a.s[d][q], ub = a.b[d][q];
-        const double unew = ub + rk * (R - g.c15 * us + a.c[d][q]);
-        a.s[d][q] = unew;
-        if (last) {
-            const double w = (xd == 0 || xd == n) ? 0.5 : 1.0;
-            const double df = ub - unew;
-            sq = w * df * df;
-            a.b[d][q] = unew;
-        }
-    }
-    if (last) {
-        const double r = block_reduce<false>(sq, sh);
-        if (threadIdx.x == 0)
-            for (int k = 0; k < 3; ++k) partials[3 * blk + k] = k == d ? r : 0.0;
-    }
-}
-
 // Error_Computation from the block partials (records of three, one sum per
 // direction); the loop control of main.cpp:898-1039 (countIter, IterNum cap,
 // divergence guard), or for PSEUDO_TIMESTEPPING = 0 the single update's norm
@@ -659,9 +549,11 @@ __global__ __launch_bounds__(1024) void k_gen_fin_pseudo(Geom g, const double *p
 // ------------------------------------------------------------ BDF2 constant
 // main.cpp:879-884 with the pressure term folded: C = (1.5/dt) u^n + (0.5/dt)
 // (u^n - u^{n-1}) - G p (p's ghosts: Neumann mirror, so G p = 0 on wall
-// faces; periodic images); in 2D then u^{n-1} <- u^n and u^k = u* = u^n.
+// faces; periodic images).  The stages then read u^n in place, and the face arrays
+// change roles instead of being copied (amr_gen_advance).
 struct Bdf2Arrays {
-    double *u[3], *up[3], *c[3], *b[3], *s[3];
+    const double *u[3], *up[3];
+    double *c[3];
     const double *p;
     int nb[3];
 };
@@ -685,10 +577,6 @@ __global__ __launch_bounds__(B) void k_gen_bdf2(Geom g, Bdf2Arrays a)
     }
     const double un = a.u[d][q], um = a.up[d][q];
     a.c[d][q] = g.c15 * un + (0.5 / g.dt) * (un - um) - gp;
-    if (!a.b[d]) return;  // 3D: the stages read u^n in place and the arrays change roles instead
-    a.up[d][q] = un;
-    a.b[d][q] = un;
-    a.s[d][q] = un;
 }
 
 // ------------------------------------------------------------ divergence
@@ -1077,13 +965,6 @@ hipError_t cells(const Ctx &c, hipStream_t s, double *const *f, double *X, const
     return hipGetLastError();
 }
 
-hipError_t flux(const Ctx &c, hipStream_t s, double *const *f, const double *X, double *T, const Ctl *guard)
-{
-    hipLaunchKernelGGL(k_gen_flux, dim3(nblk(c.g.ncell)), dim3(B), 0, s, c.g, f[0], f[1],
-                       c.g.dim == 3 ? f[2] : f[0], X, T, guard);
-    return hipGetLastError();
-}
-
 void stage3_shape(int n, int *ntx, int *nty, int *zc)
 {
     *ntx = (n + 1 + kS3X - 1) / kS3X;
@@ -1103,6 +984,35 @@ void stage3_shape(int n, int *ntx, int *nty, int *zc)
 int stage3_blocks(const Ctx &c)
 {
     return c.s3_ntx * c.s3_nty * ((c.g.n + 1 + c.s3_zc - 1) / c.s3_zc);
+}
+
+hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, const Ctl *guard)
+{
+    IterTile a{};
+    const Geom &g = c.g;
+    a.u = base[0]; a.v = base[1];
+    a.cu = c.C[0]; a.cv = c.C[1];
+    a.uo = out[0]; a.vo = out[1];
+    a.partials = c.partials;
+    a.guard = guard;
+    a.n = g.n;
+    a.su = g.n + 1;
+    a.sv = g.n;
+    a.rec = 3;
+    a.nst = g.pseudo ? 4 : 1;
+    a.expl = !g.pseudo;
+    for (int k = 0; k < 4; ++k) a.rk[k] = g.pseudo ? c.rk[k] : g.dt / 1.5;
+    a.c15 = g.c15;
+    a.iren = g.iren;
+    for (int d = 0; d < 2; ++d) {
+        a.per[d] = g.per[d];
+        a.kind[2 * d] = g.kind_lo[d];
+        a.kind[2 * d + 1] = g.kind_hi[d];
+        a.inflow[d] = g.inflow[d];
+        a.idx[d] = g.idx[d];
+        a.idx2[d] = g.idx2[d];
+    }
+    return launch_iter_tile(a, s);
 }
 
 hipError_t stage3(const Ctx &c, hipStream_t s, double *const *in, double *const *base, double *const *out, double rk,
@@ -1139,23 +1049,9 @@ hipError_t stage3(const Ctx &c, hipStream_t s, double *const *in, double *const 
     return hipGetLastError();
 }
 
-hipError_t update(const Ctx &c, hipStream_t s, double rk, int last, const Ctl *guard)
-{
-    FaceArrays a{};
-    for (int d = 0; d < 3; ++d) {
-        a.s[d] = d < c.g.dim ? c.S[d] : nullptr;
-        a.b[d] = d < c.g.dim ? c.B[d] : nullptr;
-        a.c[d] = d < c.g.dim ? c.C[d] : nullptr;
-        a.nb[d] = d < c.g.dim ? c.nb_face[d] : 0;
-    }
-    const int nb = a.nb[0] + a.nb[1] + a.nb[2];
-    hipLaunchKernelGGL(k_gen_update, dim3(nb), dim3(B), 0, s, c.g, a, c.T, rk, last, c.partials, guard);
-    return hipGetLastError();
-}
-
 hipError_t fin_pseudo(const Ctx &c, hipStream_t s, Ctl *ctl)
 {
-    const int nrec = c.g.dim == 3 ? stage3_blocks(c) : c.nb_face[0] + c.nb_face[1];
+    const int nrec = c.g.dim == 3 ? stage3_blocks(c) : iter_tile_blocks(c.g.n);
     hipLaunchKernelGGL(k_gen_fin_pseudo, dim3(1), dim3(1024), 0, s, c.g, c.partials, nrec, ctl);
     return hipGetLastError();
 }
@@ -1168,8 +1064,6 @@ hipError_t bdf2(const Ctx &c, hipStream_t s)
         a.u[d] = on ? c.U[d] : nullptr;
         a.up[d] = on ? c.Up[d] : nullptr;
         a.c[d] = on ? c.C[d] : nullptr;
-        a.b[d] = on && c.g.dim == 2 ? c.B[d] : nullptr;
-        a.s[d] = on && c.g.dim == 2 ? c.S[d] : nullptr;
         a.nb[d] = on ? c.nb_face[d] : 0;
     }
     a.p = c.p;

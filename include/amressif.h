@@ -374,12 +374,11 @@ int amressif_amr_advance(amressif_amr *amr, int nsteps, amressif_amr_stats *stat
  *   which = 5  finest-level up-leg smoother with the fused FP64 outer step (V-cycle precision)
  *   which = 6  two FP64 RK stages in one pass (stages 1-2 of a pseudo-iteration)
  *   which = 10 mixed precision: one mixed iteration in one pass (residual + tangent-linear update)
+ *   which = 11 one FP64 pseudo-iteration of four stages in one pass
  * On a 3D or periodic context (the general path), each over the whole grid:
  *   which = 7  cell velocities with their ghost layers (cont2cart)
- *   which = 8  2D: fluxTotal (QUICK convective and viscous fluxes per cell);
- *              3D: one RK4 stage
- *   which = 9  2D: stage update of every face; 3D: one RK4 stage with the
- *              pseudo-iteration's norm partials
+ *   which = 8  3D: one RK4 stage; 2D: one pseudo-iteration of four stages
+ *   which = 9  3D: one RK4 stage with the pseudo-iteration's norm partials; 2D: as 8
  * which = 3, 4 and 10 need a context created with precision = 1.
  * bytes_per_launch receives the kernel's algorithmic HBM bytes per launch. */
 int amressif_time_kernel(amressif_ctx *ctx, int which, int reps, int64_t copy_bytes, double *avg_ms,
@@ -402,6 +401,8 @@ int amressif_time_kernel(amressif_ctx *ctx, int which, int reps, int64_t copy_by
  *   which = 8  FP64 RK stages 1-2 in one pass
  *   which = 9  FP64 RK stages 3-4 in one pass (+ norm partials)
  *   which = 10 mixed iteration in one pass (residual + tangent-linear update + norm partials)
+ * (where all four stages are one launch, 8 and 9 each count it with half its
+ * time and the bytes of a two-stage pass)
  * amressif_kernel_time returns the average time per counted launch (0 if none),
  * the number of counted launches and their average algorithmic HBM bytes (the
  * bytes each launch must read and write, counted once per cell). */

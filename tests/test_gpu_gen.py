@@ -118,6 +118,15 @@ def test_2d_periodic_steps_match_oracle(bc_lo, bc_hi):
     _check(ref, ref_stats, got, stats, 2)
 
 
+@pytest.mark.parametrize("n", [4, 5, 24, 31, 288])
+@pytest.mark.parametrize("bc_lo,bc_hi", [((111, 111, 0), (111, 111, 0)), ((-135, 111, 0), (165, 111, 0))])
+def test_2d_pseudo_iteration_tile_edges(n, bc_lo, bc_hi):
+    """The one-launch 2D pseudo-iteration where its halo of 12 wraps a small
+    periodic box several times, and in the 40-row tiles (n >= 280)."""
+    ref, ref_stats, got, stats, _, _ = _run_pair(2, n, 300.0, bc_lo, bc_hi, 2, inflow=(0.5, -0.2, 0.0), amp=0.1)
+    _check(ref, ref_stats, got, stats, 2)
+
+
 def test_2d_taylor_green_matches_oracle():
     n = 64
     L = 2 * np.pi

@@ -318,6 +318,41 @@ def test_two_stage_pass_matches_four_stage_launches(n, rows, init, bc, lid):
         assert rel(p2 - p2.mean(), p4 - p4.mean()) < 1e-12, name
 
 
+@pytest.mark.parametrize("n,init,bc,lid", [
+    (4, "seeded", 0, False), (8, "seeded", 3, False), (38, "seeded", 1, False), (40, "seeded", 2, False),
+    (78, "zero", 0, True), (128, "seeded", 2, True), (279, "seeded", 0, True), (280, "seeded", 1, False),
+    (319, "seeded", 2, True), (320, "seeded", 3, False), (600, "seeded", 0, False)])
+def test_one_launch_pseudo_iteration_matches_four_stage_launches(n, init, bc, lid):
+    """The FP64 pseudo-iteration as one tile launch against four single-stage
+    launches: the same pseudo-iteration counts and the same fields to rounding,
+    below one tile (40 columns), at whole tiles (n + 1 = 80, 280, 320) and one
+    face past them, in the 8-row tiles (n <= 279) and the 40-row ones, with
+    every wall set, a lid profile, and batches that overshoot convergence (the
+    skipped launches copy the base)."""
+    api = _api()
+    prof = W.lid_profile(n) if lid else None
+
+    def run():
+        inp = api.cavity_inputs(n, 400.0, phy_bc_lo=(BCS[bc][0][0], BCS[bc][0][1], 135),
+                                phy_bc_hi=(BCS[bc][1][0], BCS[bc][1][1], 135), inflow_waveform=(0.8, -0.1, 0.0))
+        r = api.Run.from_numpy(inp, W.initial_state(n, init))
+        if prof is not None:
+            r.ctx.set_lid_profile(cuda(prof))
+        st = r.advance(4)
+        return r.fetch(), st
+
+    f4, s4 = _with_env({"AMRESSIF_STAGE_PAIR": "0"}, run)
+    f1, s1 = _with_env({"AMRESSIF_ITER_TILE": "2"}, run)
+    print(f"n={n}: pseudo-iterations {[s['pseudo_iters'] for s in s1]}, u {rel(f1['u'], f4['u']):.1e} "
+          f"v {rel(f1['v'], f4['v']):.1e}")
+    assert [s["pseudo_iters"] for s in s1] == [s["pseudo_iters"] for s in s4]
+    assert all(s["flags"] == 0 for s in s1)
+    for k in ("u", "v", "uprev"):
+        assert rel(f1[k], f4[k]) < 1e-12, k
+    p1, p4 = f1["ctx"][0, 1:-1, 1:-1], f4["ctx"][0, 1:-1, 1:-1]
+    assert rel(p1 - p1.mean(), p4 - p4.mean()) < 1e-11
+
+
 @pytest.mark.parametrize("n,rows,init,bc,lid", [
     (8, 4, "seeded", 0, False), (64, 4, "seeded", 0, False), (64, 5, "seeded", 1, False),
     (100, 16, "seeded", 2, True), (130, 7, "seeded", 0, False), (256, 16, "seeded", 3, False),
