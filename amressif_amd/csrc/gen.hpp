@@ -44,7 +44,8 @@ struct Geom {
 struct Level {
     int n;            // cells per side
     double a[3];      // 1/h_d^2 of this level
-    double *e, *r;    // correction and right-hand side (n^dim)
+    double *e, *r;    // the down leg's correction and the right-hand side (n^dim)
+    double *out;      // the up leg's (or the exact solve's) correction
     int64_t ncell;
 };
 
@@ -56,8 +57,8 @@ struct Ctx {
     double *p = nullptr, *phi = nullptr, *b = nullptr;
     Level lev[kMaxGenLevels]{};
     int nlev = 0;
-    double *pinv = nullptr;  // bottom pseudo-inverse (m x m, symmetric)
-    int mb = 0;
+    double *exact = nullptr;  // coarsest level: eigenvectors and eigenvalues of its 1D operators
+    double *phi2 = nullptr;   // the solve's iterates alternate between phi and phi2
     double *partials = nullptr;
     int64_t npartials = 0;
     int nb_face[3]{};        // blocks per face direction of a launch over every face
@@ -83,10 +84,14 @@ hipError_t divergence(const Ctx &c, hipStream_t s, double *const *faces, double 
 // which 0: div_star, rhs_sum and b's mean (the step's Poisson RHS), 1: div_new
 hipError_t fin_div(const Ctx &c, hipStream_t s, int nblocks, Ctl *ctl, int which);
 hipError_t mg_start(const Ctx &c, hipStream_t s, Ctl *ctl);
-hipError_t resid0(const Ctx &c, hipStream_t s, const Ctl *ctl, int *nblocks);
-hipError_t fin_resid(const Ctx &c, hipStream_t s, int nblocks, Ctl *ctl);
+// one V-cycle for L e = lev[0].r into lev[0].out (kernels_gen_mg.hip)
 hipError_t vcycle(const Ctx &c, hipStream_t s, const Ctl *ctl);
-// phi's mean into the control block, then u = u* - (dt/1.5) G phi and p += phi - mean
+// phi2 = phi + e, lev[0].r = (b - mean) - L phi2 and the stopping test (e null: phi2 = 0)
+hipError_t outer(const Ctx &c, hipStream_t s, const double *phi, const double *e, double *phi2, Ctl *ctl);
+int outer_blocks(int dim, int n);
+// the exact 2D solve of a level of at most 64^2 cells (kernels_mg.hip's k_tail_dct)
+hipError_t launch_exact2(hipStream_t s, const double *r, double *e, int n, const double *tab, const Ctl *ctl);
+// u = u* - (dt/1.5) G phi and p += phi - mean (the solve's)
 hipError_t project(const Ctx &c, hipStream_t s, Ctl *ctl);
 hipError_t fin_step(const Ctx &c, hipStream_t s, Ctl *ctl, amressif_step_stats *log);
 hipError_t fill(hipStream_t s, double *dst, int64_t count, double value);

@@ -69,66 +69,60 @@ int side_kind(int d, int hi, int code)
     return -3;
 }
 
-// pinv(L) = J - (J - L)^{-1}, J = 11^T/m, by Cholesky of J - L (SPD: L's
-// null space is the constants with Neumann and periodic sides alike); stored
-// transposed (column j of row i at j m + i) for the device's column reads
-bool bottom_pinv(const G::Geom &g, const G::Level &L, std::vector<double> &out)
+// Orthonormal eigenvectors Q[i][k] (row stride ld) and eigenvalues of the 1D second
+// difference a (e(i + 1) - 2 e(i) + e(i - 1)) on m cells: DCT-II vectors with Neumann
+// ends, cosines and sines of the same wave number with periodic ones.  Vector 0 is
+// the constant.
+void modes_1d(int m, double a, bool per, std::vector<double> &Q, std::vector<double> &lam)
 {
-    const int n = L.n, dim = g.dim;
-    const int m = (int)L.ncell;
-    std::vector<double> A((size_t)m * m, 0.0);
-    auto at = [&](int i, int j) -> double & { return A[(size_t)i * m + j]; };
-    for (int q = 0; q < m; ++q) {
-        const int x[3] = {q % n, (q / n) % n, dim == 3 ? q / (n * n) : 0};
-        int st = 1;
-        for (int d = 0; d < dim; ++d) {
-            for (int s = -1; s <= 1; s += 2) {
-                int y = x[d] + s;
-                if (y < 0 || y >= n) {
-                    if (!g.per[d]) continue;  // Neumann: the mirror ghost is the cell itself
-                    y = (y + n) % n;
-                }
-                const int nb = q + (y - x[d]) * st;
-                at(q, nb) += L.a[d];
-                at(q, q) -= L.a[d];
-            }
-            st *= n;
-        }
-    }
-    // J - L
-    for (int i = 0; i < m; ++i)
-        for (int j = 0; j < m; ++j) at(i, j) = 1.0 / m - at(i, j);
-    for (int j = 0; j < m; ++j) {
-        double s = at(j, j);
-        for (int k = 0; k < j; ++k) s -= at(j, k) * at(j, k);
-        if (!(s > 0)) return false;
-        const double l = std::sqrt(s);
-        at(j, j) = l;
-        for (int i = j + 1; i < m; ++i) {
-            double t = at(i, j);
-            for (int k = 0; k < j; ++k) t -= at(i, k) * at(j, k);
-            at(i, j) = t / l;
-        }
-    }
-    out.assign((size_t)m * m, 0.0);
-    std::vector<double> col(m);
-    for (int j = 0; j < m; ++j) {
-        std::fill(col.begin(), col.end(), 0.0);
-        col[j] = 1.0;
+    const double pi = 3.14159265358979323846;
+    Q.assign((size_t)m * m, 0.0);
+    lam.assign(m, 0.0);
+    for (int k = 0; k < m; ++k) {
+        const int f = per ? (k + 1) / 2 : k;  // wave number
+        double nrm = 0.0;
         for (int i = 0; i < m; ++i) {
-            double t = col[i];
-            for (int k = 0; k < i; ++k) t -= at(i, k) * col[k];
-            col[i] = t / at(i, i);
+            double v;
+            if (!per) v = std::cos(pi * (double)(((int64_t)(2 * i + 1) * f) % (4 * m)) / (2 * m));
+            else if (k % 2 == 1 || k == 0) v = std::cos(2 * pi * (double)((int64_t)i * f % m) / m);
+            else v = std::sin(2 * pi * (double)((int64_t)i * f % m) / m);
+            Q[(size_t)i * m + k] = v;
+            nrm += v * v;
         }
-        for (int i = m - 1; i >= 0; --i) {
-            double t = col[i];
-            for (int k = i + 1; k < m; ++k) t -= at(k, i) * col[k];
-            col[i] = t / at(i, i);
-        }
-        // pinv(i, j) for every i, stored at j m + i
-        for (int i = 0; i < m; ++i) out[(size_t)j * m + i] = 1.0 / m - col[i];
+        for (int i = 0; i < m; ++i) Q[(size_t)i * m + k] /= std::sqrt(nrm);
+        const double h = std::sin(pi * f / (per ? m : 2.0 * m));
+        lam[k] = -4.0 * a * h * h;
     }
-    return true;
+}
+
+// the tables of the coarsest level's exact solve (k_gen_exact3 in 3D, k_tail_dct in 2D)
+std::vector<double> exact_tables(const G::Geom &g, const G::Level &L)
+{
+    const int m = L.n;
+    std::vector<double> Q[3], lam[3], t;
+    for (int d = 0; d < g.dim; ++d) modes_1d(m, L.a[d], g.per[d] != 0, Q[d], lam[d]);
+    if (g.dim == 3) {
+        const int ld = 24;
+        t.assign((size_t)6 * m * ld + (size_t)m * m * m, 0.0);
+        for (int d = 0; d < 3; ++d) {
+            double *q = t.data() + (size_t)2 * d * m * ld, *qt = q + (size_t)m * ld;
+            for (int i = 0; i < m; ++i)
+                for (int k = 0; k < m; ++k) q[i * ld + k] = qt[k * ld + i] = Q[d][(size_t)i * m + k];
+        }
+        double *dinv = t.data() + (size_t)6 * m * ld;
+        for (int q = 1; q < m * m * m; ++q)  // the constant mode's stays 0
+            dinv[q] = 1.0 / (lam[0][q % m] + lam[1][(q / m) % m] + lam[2][q / (m * m)]);
+        return t;
+    }
+    const int ld = 64;
+    t.assign((size_t)3 * ld * ld, 0.0);
+    for (int i = 0; i < m; ++i)
+        for (int k = 0; k < m; ++k) {
+            t[i * ld + k] = Q[0][(size_t)i * m + k];
+            t[ld * ld + i * ld + k] = Q[1][(size_t)i * m + k];
+            t[2 * ld * ld + i * ld + k] = i + k == 0 ? 0.0 : 1.0 / (lam[0][k] + lam[1][i]);
+        }
+    return t;
 }
 
 int poll(amressif_ctx *ctx)
@@ -227,8 +221,9 @@ int amr_gen_create(amressif_ctx *ctx)
         g.nf[d] = (int64_t)ext[0] * ext[1] * ext[2];
         gc.nb_face[d] = (int)((g.nf[d] + G::kBlock - 1) / G::kBlock);
     }
-    // multigrid hierarchy: halve while the side is even and the level holds
-    // more than 512 cells; the coarsest level's dense pseudo-inverse
+    // multigrid hierarchy: halve while the side is even and the level holds more
+    // than 512 cells; the first level of at most 20 (3D) or 64 (2D) cells per side is
+    // solved exactly and ends it
     {
         int nl = n, l = 0;
         for (;;) {
@@ -244,10 +239,10 @@ int amr_gen_create(amressif_ctx *ctx)
             nl /= 2;
         }
         gc.nlev = l;
-        gc.mb = (int)gc.lev[l - 1].ncell;
         if (gc.lev[l - 1].ncell > 1024)
             return gfail(ctx, AMRESSIF_ERR_UNSUPPORTED,
                          "coarsest multigrid level above 1024 cells (n_cell = m 2^k with m^dim > 1024, m odd)");
+        while (gc.nlev > 1 && gc.lev[gc.nlev - 2].n <= (dim == 3 ? 20 : 64)) gc.nlev -= 1;
     }
     if (dim == 3) {
         G::stage3_shape(n, &gc.s3_ntx, &gc.s3_nty, &gc.s3_zc);
@@ -264,20 +259,19 @@ int amr_gen_create(amressif_ctx *ctx)
         GALLOC(&gc.B[d], g.nf[d]); GALLOC(&gc.S[d], g.nf[d]);
     }
     GALLOC(&gc.X, (size_t)g.xs * dim);
-    GALLOC(&gc.p, cellsz); GALLOC(&gc.phi, cellsz); GALLOC(&gc.b, cellsz);
+    GALLOC(&gc.p, cellsz); GALLOC(&gc.phi, cellsz); GALLOC(&gc.phi2, cellsz); GALLOC(&gc.b, cellsz);
     for (int l = 0; l < gc.nlev; ++l) {
-        GALLOC(&gc.lev[l].e, (size_t)gc.lev[l].ncell);
+        if (l + 1 < gc.nlev) GALLOC(&gc.lev[l].e, (size_t)gc.lev[l].ncell);
         GALLOC(&gc.lev[l].r, (size_t)gc.lev[l].ncell);
+        GALLOC(&gc.lev[l].out, (size_t)gc.lev[l].ncell);
     }
-    gc.npartials = std::max<int64_t>(2 * ((g.ncell + G::kBlock - 1) / G::kBlock),
+    gc.npartials = std::max<int64_t>(std::max<int64_t>(2 * ((g.ncell + G::kBlock - 1) / G::kBlock), 2 * G::outer_blocks(dim, n)),
                                      3 * (int64_t)(dim == 3 ? G::stage3_blocks(gc) : amr::iter_tile_blocks(n))) + 64;
     GALLOC(&gc.partials, (size_t)gc.npartials);
     {
-        std::vector<double> pinv;
-        if (!bottom_pinv(g, gc.lev[gc.nlev - 1], pinv))
-            return gfail(ctx, AMRESSIF_ERR_ARG, "bottom factorisation failed");
-        GALLOC(&gc.pinv, pinv.size());
-        GCHK(hipMemcpy(gc.pinv, pinv.data(), pinv.size() * sizeof(double), hipMemcpyHostToDevice));
+        const std::vector<double> tab = exact_tables(g, gc.lev[gc.nlev - 1]);
+        GALLOC(&gc.exact, tab.size());
+        GCHK(hipMemcpy(gc.exact, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
     }
     GALLOC(&c.ctl, 1);
     {
@@ -595,21 +589,21 @@ int amr_gen_advance(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats)
         GCHK(G::divergence(gc, c.stream, gc.S, gc.b, &nb));
         GCHK(G::fin_div(gc, c.stream, nb, c.ctl, 0));
         GCHK(G::mg_start(gc, c.stream, c.ctl));
-        GCHK(G::fill(c.stream, gc.phi, g.ncell, 0.0));  // phi0 = 0 (poisson.cpp:63)
-        {
-            int done = 0, batch = std::max(1, gc.last_V);
+        {   // from phi0 = 0 (poisson.cpp:63); the iterate alternates between phi2 (even cycles) and phi
+            int done = 0, batch = std::max(1, gc.last_V), k = 0;
+            auto iter = [&](int q) { return (q & 1) ? gc.phi : gc.phi2; };
+            GCHK(G::outer(gc, c.stream, nullptr, nullptr, iter(0), c.ctl));
             while (!done) {
-                for (int it = 0; it < batch; ++it) {
-                    int nr = 0;
-                    GCHK(G::resid0(gc, c.stream, c.ctl, &nr));
-                    GCHK(G::fin_resid(gc, c.stream, nr, c.ctl));
+                for (int it = 0; it < batch; ++it, ++k) {
                     GCHK(G::vcycle(gc, c.stream, c.ctl));
+                    GCHK(G::outer(gc, c.stream, iter(k), gc.lev[0].out, iter(k + 1), c.ctl));
                 }
                 if (int rc = poll(ctx)) return rc;
                 done = c.ctl_host->mg_done;
                 batch = 2;
             }
-            gc.last_V = std::max(1, c.ctl_host->mg_iters + 1);
+            gc.last_V = std::max(1, c.ctl_host->mg_iters);
+            if (c.ctl_host->mg_iters % 2 == 0) std::swap(gc.phi, gc.phi2);
         }
         // ---- projection, p += phi - mean, divergence of u^{n+1}
         GCHK(G::project(gc, c.stream, c.ctl));

@@ -11,10 +11,8 @@
 // (1.5/dt) u* + C), the BDF2 constant C holding -G p (momentum.cpp:68-87,
 // fn_rhs.cpp:8-68); on the last stage the Error_Computation partials
 // (utilities.cpp:421-493).  k_gen_cells writes the cell velocities for output.
-// Then the Poisson RHS (fn_rhs.cpp:71-125), a geometric V-cycle iteration with
-// red-black Gauss-Seidel on Neumann / periodic neighbours and a dense
-// pseudo-inverse bottom (poisson.cpp:41-186), and the projection
-// (poisson.cpp:192-392).  Blocks are handed to the XCDs in contiguous ranges
+// Then the Poisson RHS (fn_rhs.cpp:71-125), the multigrid solve
+// (kernels_gen_mg.hip), and the projection (poisson.cpp:192-392).  Blocks are handed to the XCDs in contiguous ranges
 // (xcd_block), so the rows and planes a stencil shares sit in one L2.
 #include "device_common.hpp"
 #include "gen.hpp"
@@ -616,17 +614,16 @@ __global__ __launch_bounds__(B) void k_gen_div(Geom g, const double *f0, const d
     }
 }
 
-__global__ __launch_bounds__(B) void k_gen_fin_div(const double *partials, int nb, Ctl *ctl, double ncell, int which)
+__global__ __launch_bounds__(1024) void k_gen_fin_div(const double *partials, int nb, Ctl *ctl, double ncell, int which)
 {
-    __shared__ double sh[B / 64];
-    double m = 0.0, s = 0.0;
-    for (int k = threadIdx.x; k < nb; k += B) {
-        const double v = partials[2 * k];
-        m = (v > m || v != v) ? v : m;
-        s += partials[2 * k + 1];
-    }
-    m = block_reduce<true>(m, sh);
-    s = block_reduce<false>(s, sh);
+    __shared__ double sh[32];
+    double v[2] = {0.0, 0.0};
+    for_records<2, 2>(partials, nb, [&](const double *a) {
+        v[0] = (a[0] > v[0] || a[0] != a[0]) ? a[0] : v[0];
+        v[1] += a[1];
+    });
+    block_reduce_n<1u>(v, sh);
+    const double m = v[0], s = v[1];
     if (threadIdx.x != 0) return;
     if (which == 0) {
         ctl->div_star = m;
@@ -637,183 +634,12 @@ __global__ __launch_bounds__(B) void k_gen_fin_div(const double *partials, int n
     }
 }
 
-// ------------------------------------------------------------ multigrid
-// Laplacian of e at cell x of a level (n cells per side, a = 1/h^2): Neumann
-// wall neighbours are the cell itself (their term drops), periodic ones wrap
-__device__ __forceinline__ double lap(const Geom &g, const Level &L, const double *e, const int *x, int64_t q)
-{
-    const int n = L.n;
-    const double ec = e[q];
-    double s = 0.0;
-    int64_t st = 1;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (d >= g.dim) break;
-        const int64_t lo = x[d] > 0 ? q - st : (g.per[d] ? q + st * (n - 1) : q);
-        const int64_t hi = x[d] < n - 1 ? q + st : (g.per[d] ? q - st * (n - 1) : q);
-        s += (e[hi] - 2.0 * ec + e[lo]) * L.a[d];
-        st *= n;
-    }
-    return s;
-}
-
-__device__ __forceinline__ void lcoords(const Geom &g, int n, int64_t q, int *x)
-{
-    split3(q, n, n, x);
-    if (g.dim != 3) x[2] = 0;
-}
-
+// ------------------------------------------------------------ Poisson control
 __global__ void k_gen_mg_start(Ctl *ctl)
 {
     ctl->mg_done = 0;
     ctl->mg_iters = 0;
     ctl->mg_started = 0;
-}
-
-// r0 = (b - mean b) - L phi and its max-norm partials
-__global__ __launch_bounds__(B) void k_gen_resid0(Geom g, Level L, const double *phi, const double *b,
-                                                  double *partials, const Ctl *ctl)
-{
-    __shared__ double sh[B / 64];
-    if (ctl->mg_done) return;
-    const int64_t q = gid();
-    double m = 0.0;
-    if (q < L.ncell) {
-        int x[3];
-        lcoords(g, L.n, q, x);
-        const double r = (b[q] - ctl->b_mean) - lap(g, L, phi, x, q);
-        L.r[q] = r;
-        m = fabs(r);
-        if (r != r) m = r;
-    }
-    m = block_reduce<true>(m, sh);
-    if (threadIdx.x == 0) partials[blockIdx.x] = m;
-}
-
-// the stopping test ||r||inf <= max(tol_abs, tol_rel ||b - mean||inf)
-// (poisson.cpp:181-182); the first residual (phi = 0) is b - mean itself
-__global__ __launch_bounds__(B) void k_gen_fin_resid(const double *partials, int nb, Ctl *ctl)
-{
-    __shared__ double sh[B / 64];
-    if (ctl->mg_done) return;
-    double m = 0.0;
-    for (int k = threadIdx.x; k < nb; k += B) {
-        const double v = partials[k];
-        m = (v > m || v != v) ? v : m;
-    }
-    m = block_reduce<true>(m, sh);
-    if (threadIdx.x != 0) return;
-    if (!ctl->mg_started) {
-        ctl->b_norm = m;
-        ctl->mg_started = 1;
-    }
-    ctl->res_norm = m;
-    const double thr = fmax(ctl->tol_abs, ctl->tol_rel * ctl->b_norm);
-    if (m <= thr || !(m == m)) ctl->mg_done = 1;
-    else if (ctl->mg_iters >= ctl->mg_max_iter) {
-        ctl->flags |= AMRESSIF_FLAG_MG_CAP;
-        ctl->mg_done = 1;
-    } else ctl->mg_iters += 1;
-}
-
-// red-black Gauss-Seidel sweep of L e = r; first: e = 0 before the sweep (the
-// first red sweep reads no neighbour)
-__global__ __launch_bounds__(B) void k_gen_gsrb(Geom g, Level L, int color, int first, const Ctl *ctl)
-{
-    if (ctl->mg_done) return;
-    const int64_t q = gid();
-    if (q >= L.ncell) return;
-    int x[3];
-    lcoords(g, L.n, q, x);
-    if (((x[0] + x[1] + x[2]) & 1) != color) return;
-    const int n = L.n;
-    double off = 0.0, diag = 0.0;
-    int64_t st = 1;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (d >= g.dim) break;
-        const bool haslo = x[d] > 0 || g.per[d], hashi = x[d] < n - 1 || g.per[d];
-        if (haslo) {
-            if (!first) off += L.a[d] * L.e[x[d] > 0 ? q - st : q + st * (n - 1)];
-            diag += L.a[d];
-        }
-        if (hashi) {
-            if (!first) off += L.a[d] * L.e[x[d] < n - 1 ? q + st : q - st * (n - 1)];
-            diag += L.a[d];
-        }
-        st *= n;
-    }
-    L.e[q] = (off - L.r[q]) / diag;
-}
-
-// r_c = 2^-dim sum over the children of (r - L e)
-__global__ __launch_bounds__(B) void k_gen_restrict(Geom g, Level F, Level Cl, const Ctl *ctl)
-{
-    if (ctl->mg_done) return;
-    const int64_t q = gid();
-    if (q >= Cl.ncell) return;
-    int c[3];
-    lcoords(g, Cl.n, q, c);
-    double s = 0.0;
-    const int nz = g.dim == 3 ? 2 : 1;
-    for (int dz = 0; dz < nz; ++dz)
-        for (int dy = 0; dy < 2; ++dy)
-#pragma unroll
-            for (int dx = 0; dx < 2; ++dx) {
-                int f[3] = {2 * c[0] + dx, 2 * c[1] + dy, g.dim == 3 ? 2 * c[2] + dz : 0};
-                const int64_t k = f[0] + (int64_t)F.n * (f[1] + (int64_t)F.n * f[2]);
-                s += F.r[k] - lap(g, F, F.e, f, k);
-            }
-    Cl.r[q] = (g.dim == 3 ? 0.125 : 0.25) * s;
-}
-
-// cell-centred (bi/tri)linear prolongation: per direction 3/4 of the coarse
-// cell and 1/4 of its neighbour on the fine cell's side (the periodic image,
-// or the cell itself past a wall: the Neumann mirror)
-__global__ __launch_bounds__(B) void k_gen_prolong(Geom g, Level F, Level Cl, const Ctl *ctl)
-{
-    if (ctl->mg_done) return;
-    const int64_t q = gid();
-    if (q >= F.ncell) return;
-    int f[3];
-    lcoords(g, F.n, q, f);
-    int c[3] = {0, 0, 0}, nb[3] = {0, 0, 0};
-    const int m = Cl.n;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (d >= g.dim) break;
-        c[d] = f[d] >> 1;
-        int t = (f[d] & 1) ? c[d] + 1 : c[d] - 1;
-        if (t < 0 || t >= m) t = g.per[d] ? (t + m) % m : c[d];
-        nb[d] = t;
-    }
-    double s = 0.0;
-    const int corners = 1 << g.dim;
-    for (int k = 0; k < corners; ++k) {
-        const int x = (k & 1) ? nb[0] : c[0], y = (k & 2) ? nb[1] : c[1], z = (k & 4) ? nb[2] : c[2];
-        const double w = ((k & 1) ? 0.25 : 0.75) * ((k & 2) ? 0.25 : 0.75) * (g.dim == 3 ? ((k & 4) ? 0.25 : 0.75) : 1.0);
-        s += w * Cl.e[x + (int64_t)m * (y + (int64_t)m * z)];
-    }
-    F.e[q] += s;
-}
-
-// e = pinv r on the coarsest level (pinv symmetric, read by columns)
-__global__ __launch_bounds__(B) void k_gen_bottom(Level L, const double *pinv, const Ctl *ctl)
-{
-    if (ctl->mg_done) return;
-    const int64_t i = (int64_t)blockIdx.x * B + threadIdx.x;
-    const int64_t m = L.ncell;
-    if (i >= m) return;
-    double s = 0.0;
-    for (int64_t j = 0; j < m; ++j) s += pinv[j * m + i] * L.r[j];
-    L.e[i] = s;
-}
-
-__global__ __launch_bounds__(B) void k_gen_correct(Level L, double *phi, const Ctl *ctl)
-{
-    if (ctl->mg_done) return;
-    const int64_t q = gid();
-    if (q < L.ncell) phi[q] += L.e[q];
 }
 
 // ------------------------------------------------------------ projection
@@ -1081,52 +907,13 @@ hipError_t divergence(const Ctx &c, hipStream_t s, double *const *f, double *b, 
 
 hipError_t fin_div(const Ctx &c, hipStream_t s, int nblocks, Ctl *ctl, int which)
 {
-    hipLaunchKernelGGL(k_gen_fin_div, dim3(1), dim3(B), 0, s, c.partials, nblocks, ctl, (double)c.g.ncell, which);
+    hipLaunchKernelGGL(k_gen_fin_div, dim3(1), dim3(1024), 0, s, c.partials, nblocks, ctl, (double)c.g.ncell, which);
     return hipGetLastError();
 }
 
 hipError_t mg_start(const Ctx &c, hipStream_t s, Ctl *ctl)
 {
     hipLaunchKernelGGL(k_gen_mg_start, dim3(1), dim3(1), 0, s, ctl);
-    return hipGetLastError();
-}
-
-hipError_t resid0(const Ctx &c, hipStream_t s, const Ctl *ctl, int *nblocks)
-{
-    *nblocks = nblk(c.lev[0].ncell);
-    hipLaunchKernelGGL(k_gen_resid0, dim3(*nblocks), dim3(B), 0, s, c.g, c.lev[0], c.phi, c.b, c.partials, ctl);
-    return hipGetLastError();
-}
-
-hipError_t fin_resid(const Ctx &c, hipStream_t s, int nblocks, Ctl *ctl)
-{
-    hipLaunchKernelGGL(k_gen_fin_resid, dim3(1), dim3(B), 0, s, c.partials, nblocks, ctl);
-    return hipGetLastError();
-}
-
-hipError_t vcycle(const Ctx &c, hipStream_t s, const Ctl *ctl)
-{
-    const int L = c.nlev;
-    for (int l = 0; l + 1 < L; ++l) {
-        const Level &F = c.lev[l];
-        const dim3 gr(nblk(F.ncell));
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 0, 1, ctl);
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 1, 0, ctl);
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 0, 0, ctl);
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 1, 0, ctl);
-        hipLaunchKernelGGL(k_gen_restrict, dim3(nblk(c.lev[l + 1].ncell)), dim3(B), 0, s, c.g, F, c.lev[l + 1], ctl);
-    }
-    hipLaunchKernelGGL(k_gen_bottom, dim3(nblk(c.lev[L - 1].ncell)), dim3(B), 0, s, c.lev[L - 1], c.pinv, ctl);
-    for (int l = L - 2; l >= 0; --l) {
-        const Level &F = c.lev[l];
-        const dim3 gr(nblk(F.ncell));
-        hipLaunchKernelGGL(k_gen_prolong, gr, dim3(B), 0, s, c.g, F, c.lev[l + 1], ctl);
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 0, 0, ctl);
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 1, 0, ctl);
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 0, 0, ctl);
-        hipLaunchKernelGGL(k_gen_gsrb, gr, dim3(B), 0, s, c.g, F, 1, 0, ctl);
-    }
-    hipLaunchKernelGGL(k_gen_correct, dim3(nblk(c.lev[0].ncell)), dim3(B), 0, s, c.lev[0], c.phi, ctl);
     return hipGetLastError();
 }
 
@@ -1140,7 +927,6 @@ hipError_t phi_mean(const Ctx &c, hipStream_t s, Ctl *ctl)
 
 hipError_t project(const Ctx &c, hipStream_t s, Ctl *ctl)
 {
-    if (hipError_t e = phi_mean(c, s, ctl)) return e;
     ProjArrays a{};
     for (int d = 0; d < 3; ++d) {
         const bool on = d < c.g.dim;

@@ -22,6 +22,7 @@
 // solve, run inside one workgroup (k_tail); then one kernel applies the
 // correction in FP64 and forms the next residual and its norm partials.
 #include "device_common.hpp"
+#include "gen.hpp"
 #include "internal.hpp"
 
 #include <algorithm>
@@ -2000,5 +2001,14 @@ hipError_t launch_smooth_fine(const Ctx &c, int kind, double *scratch_phi)
     return c.in.precision == AMRESSIF_MIXED ? smooth_probe<float>(c, kind, L.r32b, scratch_phi)
                                             : smooth_probe<double>(c, kind, L.rb, scratch_phi);
 }
+
+namespace gen {
+hipError_t launch_exact2(hipStream_t s, const double *r, double *e, int n, const double *tab, const Ctl *ctl)
+{
+    if (n > kDct) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_tail_dct<double, true, 16>), dim3(1), dim3(1024), 0, s, r, n, e, n, n, tab, ctl);
+    return hipGetLastError();
+}
+}  // namespace gen
 
 }  // namespace amr
