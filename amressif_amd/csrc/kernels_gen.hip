@@ -323,13 +323,17 @@ __global__ __launch_bounds__(64 * kS3W) void k_gen_stage3(Geom g, Stage3 a, cons
     if (LAST)
 #pragma unroll
         for (int d = 0; d < 3; ++d) shS[d][threadIdx.x] = 0.0;
-    // one face at position q along d: R from T on its two sides (wall faces: 0, or in the explicit form half
-    // of the inner T); e = C - (1.5/dt) u*
-    auto face = [&](int d, int q, double tl, double tr, double base, double e) {
-        const bool end = q == 0 || q == n;
-        double R = 0.5 * (tl + tr);
-        if (end && !g.per[d]) R = g.pseudo ? 0.0 : 0.5 * (q == 0 ? tr : tl);
-        const double unew = base + a.rk * (R + e);
+    // one face at position q along d from T on its two sides: u^k + rk (R + e), e = C - (1.5/dt) u*, R = (tl + tr)/2;
+    // at wall faces R = 0, in the explicit form half of the inner T (ends: whether this wave, row or plane
+    // can hold one; the empty asm keeps their selects out of the others' path)
+    const double rkh = 0.5 * a.rk;
+    auto face = [&](int d, bool ends, int q, double tl, double tr, double base, double e) {
+        const double uw = base + a.rk * e;
+        double unew = uw + rkh * (tl + tr);
+        if (ends && !g.per[d]) {
+            if (!LAST) asm volatile("");  // (with the norm it would spill)
+            if (q == 0 || q == n) unew = g.pseudo ? uw : uw + rkh * (q == 0 ? tr : tl);
+        }
         return unew;
     };
     auto norm = [&](int q, bool on, double base, double unew) {
@@ -413,7 +417,7 @@ __global__ __launch_bounds__(64 * kS3W) void k_gen_stage3(Geom g, Stage3 a, cons
                     for (int c = 0; c < 3; ++c) {
                         const double D = (X0[q][c] - 2.0 * X1[q][c]) + X2[q][c];
                         const double F = face_flux(f, X0[q][c], X1[q][c], dz[q][c], D);
-                        T[q][c] = (fz[q][c] - F) + a.kv[2] * dz[q][c];
+                        T[q][c] = a.kv[2] * dz[q][c] + (fz[q][c] - F);
                         fz[q][c] = F;
                         dz[q][c] = D;
                     }
@@ -423,9 +427,9 @@ __global__ __launch_bounds__(64 * kS3W) void k_gen_stage3(Geom g, Stage3 a, cons
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
                         const double X = X0[q][c], xm = lane_prev(X);
-                        const double D = (xm - 2.0 * X) + lane_next(X);
+                        const double D = -2.0 * X + (xm + lane_next(X));
                         const double F = face_flux(f, xm, X, lane_prev(D), D);
-                        T[q][c] += (F - lane_next(F)) + a.kv[0] * D;
+                        T[q][c] = a.kv[0] * D + ((T[q][c] + F) - lane_next(F));
                     }
                 }
             }
@@ -440,17 +444,17 @@ __global__ __launch_bounds__(64 * kS3W) void k_gen_stage3(Geom g, Stage3 a, cons
                     const double Fs = face_flux(fs, s1, XA, (s2 - 2.0 * s1) + XA, DA);
                     const double Fm = face_flux(fm, XA, XB, DA, DB);
                     const double Fn = face_flux(fn, XB, n1, DB, (XB - 2.0 * n1) + n2);
-                    T[0][c] += (Fs - Fm) + a.kv[1] * DA;
-                    T[1][c] += (Fm - Fn) + a.kv[1] * DB;
+                    T[0][c] = a.kv[1] * DA + ((T[0][c] + Fs) - Fm);
+                    T[1][c] = a.kv[1] * DB + ((T[1][c] + Fm) - Fn);
                 }
             }
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
-                ru[q] = face(0, i, lane_prev(T[q][0]), T[q][0], cur.ub[q], cur.uc[q] - g.c15 * pu[q]);
-                rw[q] = face(2, z, tw[q], T[q][2], cur.wb[q], cur.wc[q] - g.c15 * w0[q]);
+                ru[q] = face(0, xedge, i, lane_prev(T[q][0]), T[q][0], cur.ub[q], cur.uc[q] - g.c15 * pu[q]);
+                rw[q] = face(2, z == 0 || z == n, z, tw[q], T[q][2], cur.wb[q], cur.wc[q] - g.c15 * w0[q]);
             }
-            rv[0] = face(1, y, shT[bf][r - 1][lane], tv[0], vbl, vel);
-            rv[1] = face(1, y + 1, T[0][1], T[1][1], cur.vb[1], cur.vc[1] - g.c15 * pv[1]);
+            rv[0] = face(1, y == 0 || y == n, y, shT[bf][r - 1][lane], tv[0], vbl, vel);
+            rv[1] = face(1, y + 1 == 0 || y + 1 == n, y + 1, T[0][1], T[1][1], cur.vb[1], cur.vc[1] - g.c15 * pv[1]);
             if (LAST && z >= z0) {
                 shS[0][threadIdx.x] += norm(i, fu[0] != kNone && z < n, cur.ub[0], ru[0]) +
                                        norm(i, fu[1] != kNone && z < n, cur.ub[1], ru[1]);
@@ -484,7 +488,7 @@ __global__ __launch_bounds__(64 * kS3W) void k_gen_stage3(Geom g, Stage3 a, cons
         shT[z1 & 1][r][lane] = tv[1];
         __syncthreads();
         if (rowT) {
-            rv[0] = face(1, y, shT[z1 & 1][r - 1][lane], tv[0], vbl, vel);
+            rv[0] = face(1, y == 0 || y == n, y, shT[z1 & 1][r - 1][lane], tv[0], vbl, vel);
             if (LAST) shS[1][threadIdx.x] += norm(y, fv[0] != kNone, vbl, rv[0]);
             st(plane(a.o[1], (unsigned)(z1 - 1) * su, su), fv[0], rv[0]);
         }

@@ -167,6 +167,16 @@ def test_3d_stage_kernel_tile_edges(n, bc_lo, bc_hi):
     _check(ref, ref_stats, got, stats, 3)
 
 
+@pytest.mark.parametrize("n,bc_lo,bc_hi", [
+    (72, (135, 135, 135), (135, 165, 135)), (72, (111, 135, 111), (111, 165, 111)),
+    (96, (135, 111, 135), (135, 111, 165)), (112, (111, 111, 111), (111, 111, 111))])
+def test_3d_marching_multigrid_legs(n, bc_lo, bc_hi):
+    """Sizes whose finest multigrid legs march along z (above 64 cells per side), with partial tiles of 52 x 20
+    and 56 x 24 columns, walls and wraps; 72 ends in an exact level of 18^3, 112 of 14^3 (96: 12^3)."""
+    ref, ref_stats, got, stats, _, _ = _run_pair(3, n, 500.0, bc_lo, bc_hi, 1, inflow=(0.5, 0.0, 0.2), amp=0.05)
+    _check(ref, ref_stats, got, stats, 3)
+
+
 @pytest.mark.parametrize("dim", [2, 3])
 def test_explicit_time_marching_matches_oracle(dim):
     bc_lo = (111, 135, 135)
