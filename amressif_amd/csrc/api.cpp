@@ -389,7 +389,10 @@ int mg_loop(amressif_ctx *ctx, bool warm, bool center, const double *us, const d
 // two-term Neumann series of the inverse Jacobian (iterative refinement of the
 // implicit BDF2 system), or the RK4 recursion to first order in the Jacobian.
 int advance_impl(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats, amressif_tape *tape);
-int launch_pseudo_iteration(amressif_ctx *ctx, int it, int *nb);
+int launch_pseudo_iteration(amressif_ctx *ctx, int it, int *nb, bool chained);
+// Pseudo-iterations run as one launch each take the norm of the one before
+// themselves: only a batch's last launch needs the finalizer
+bool iterations_chain(const Ctx &c) { return c.in.precision != AMRESSIF_MIXED && amr::iter_tile_wanted(c); }
 }  // namespace
 
 // BDF2 history and the RK4 dual-time pseudo-iterations of one step
@@ -444,10 +447,12 @@ int amr_momentum_begin(amressif_ctx *ctx, bool bdf_ready, int *launched, bool re
     }
     const int target = std::min(std::max(1, c.last_P), c.in.IterNum + 1);
     for (*launched = 0; *launched < target; ++*launched) {
-        if (int rc = launch_pseudo_iteration(ctx, *launched, &nb)) return rc;
+        const bool chain = iterations_chain(c), last = *launched == target - 1;
+        if (int rc = launch_pseudo_iteration(ctx, *launched, &nb, chain && *launched > 0)) return rc;
         // with the one-pass mixed iteration, the batch's last finalizer also
         // starts the Poisson phase enqueued behind it (mg_run then skips k_mg_start)
-        HIPCHK(amr::launch_fin_pseudo(c, nb, c.mp_spec && *launched == target - 1 ? 1 : 0));
+        if (!chain) HIPCHK(amr::launch_fin_pseudo(c, nb, c.mp_spec && last ? 1 : 0));
+        else if (last) HIPCHK(amr::launch_fin_pseudo(c, nb, 0, *launched));
     }
     return 0;
 }
@@ -458,10 +463,12 @@ int amr_momentum_finish(amressif_ctx *ctx, int launched)
     const int cap = c.in.IterNum + 1;
     int target = launched, nb = 0;
     for (;;) {
-        while (launched < target && launched < cap) {
-            if (int rc = launch_pseudo_iteration(ctx, launched, &nb)) return rc;
-            HIPCHK(amr::launch_fin_pseudo(c, nb));
-            ++launched;
+        const bool chain = iterations_chain(c);
+        const int first = launched, end = std::min(target, cap);
+        for (; launched < end; ++launched) {
+            if (int rc = launch_pseudo_iteration(ctx, launched, &nb, chain && launched > first)) return rc;
+            if (!chain) HIPCHK(amr::launch_fin_pseudo(c, nb));
+            else if (launched == end - 1) HIPCHK(amr::launch_fin_pseudo(c, nb, 0, launched));
         }
         if (int rc = poll(ctx)) return rc;
         if (c.ctl_host->mom_done || launched >= cap) break;
@@ -493,7 +500,7 @@ namespace {
 // the output of the step's k-th k_mixed_pair launch: S1 for even k, S2 for odd
 double *const *mp_out(const Ctx &c, int k) { return k % 2 == 0 ? c.S1 : c.S2; }
 
-int launch_pseudo_iteration(amressif_ctx *ctx, int it, int *nb)
+int launch_pseudo_iteration(amressif_ctx *ctx, int it, int *nb, bool chained)
 {
     Ctx &c = ctx->c;
     if (c.in.precision == AMRESSIF_MIXED) {
@@ -546,6 +553,8 @@ int launch_pseudo_iteration(amressif_ctx *ctx, int it, int *nb)
     if (amr::iter_tile_wanted(c)) {
         // u^k into S1, then S1 becomes u^k (a launch skipped after convergence copies u^k to S1)
         a.uo = c.S1[0]; a.vo = c.S1[1];
+        a.it = it;
+        a.chained = chained;
         // (it moves 48 B per cell: u^k, v^k, c_u, c_v in, u^{k+1}, v^{k+1} out; its record keeps the
         // bytes of the two two-stage passes it counts as)
         HIPCHK(amr::kprof_begin(c, amr::KP_ITER, amr::KL_MOM, it, 2 * 64.0 * (double)c.g.n * c.g.n));

@@ -69,15 +69,17 @@ struct Ctx {
 // ---- launchers (kernels_gen.hip); every guarded kernel returns at once once
 // its loop's flag in the control block is set
 hipError_t cells(const Ctx &c, hipStream_t s, double *const *faces, double *X, const Ctl *guard);
-// 2D: one pseudo-iteration (or the explicit update), out <- the last stage from base; with its norm partials
-hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, const Ctl *guard);
+// 2D: the step's pseudo-iteration `it` (or the explicit update), out <- the last stage from base, with its norm
+// partials; chained: it also takes the norm of the launch before and ends the loop
+hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, int it, bool chained,
+                      Ctl *ctl);
 // 3D: one RK4 stage in one pass, out <- base + rk (R(in) - c15 in + C); out
 // aliases neither in nor base.  last: the norm partials of base - out as well
 hipError_t stage3(const Ctx &c, hipStream_t s, double *const *in, double *const *base, double *const *out, double rk,
                   int last, const Ctl *guard);
 void stage3_shape(int n, int *ntx, int *nty, int *zc);
 int stage3_blocks(const Ctx &c);
-hipError_t fin_pseudo(const Ctx &c, hipStream_t s, Ctl *ctl);
+hipError_t fin_pseudo(const Ctx &c, hipStream_t s, int it, Ctl *ctl);
 hipError_t bdf2(const Ctx &c, hipStream_t s);
 // b = (1.5/dt) D(faces) (b may be null: the norm only); partials of max|D|, sum b
 hipError_t divergence(const Ctx &c, hipStream_t s, double *const *faces, double *b, int *nblocks);

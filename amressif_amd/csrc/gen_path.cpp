@@ -266,7 +266,7 @@ int amr_gen_create(amressif_ctx *ctx)
         GALLOC(&gc.lev[l].out, (size_t)gc.lev[l].ncell);
     }
     gc.npartials = std::max<int64_t>(std::max<int64_t>(2 * ((g.ncell + G::kBlock - 1) / G::kBlock), 2 * G::outer_blocks(dim, n)),
-                                     3 * (int64_t)(dim == 3 ? G::stage3_blocks(gc) : amr::iter_tile_blocks(n))) + 64;
+                                     3 * (int64_t)(dim == 3 ? G::stage3_blocks(gc) : 2 * amr::iter_tile_blocks(n))) + 64;
     GALLOC(&gc.partials, (size_t)gc.npartials);
     {
         const std::vector<double> tab = exact_tables(g, gc.lev[gc.nlev - 1]);
@@ -553,8 +553,8 @@ int amr_gen_advance(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats)
         int count = 1;
         if (!g.pseudo) {
             if (dim3) GCHK(G::stage3(gc, c.stream, gc.U, gc.U, iter_out(1), g.dt / 1.5, 1, c.ctl));
-            else GCHK(G::iteration2(gc, c.stream, gc.U, iter_out(1), c.ctl));
-            GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
+            else GCHK(G::iteration2(gc, c.stream, gc.U, iter_out(1), 0, false, c.ctl));
+            GCHK(G::fin_pseudo(gc, c.stream, 0, c.ctl));
         } else {
             int done = 0, batch = std::max(1, gc.last_P), k = 0;
             while (!done) {
@@ -566,9 +566,10 @@ int amr_gen_advance(amressif_ctx *ctx, int nsteps, amressif_step_stats *stats)
                         GCHK(G::stage3(gc, c.stream, out, base, scratch, gc.rk[2], 0, c.ctl));
                         GCHK(G::stage3(gc, c.stream, scratch, base, out, gc.rk[3], 1, c.ctl));
                     } else {
-                        GCHK(G::iteration2(gc, c.stream, base, out, c.ctl));
+                        // each launch takes the norm of the one before: the finalizer follows the batch
+                        GCHK(G::iteration2(gc, c.stream, base, out, k, it > 0, c.ctl));
                     }
-                    GCHK(G::fin_pseudo(gc, c.stream, c.ctl));
+                    if (dim3 || it == batch - 1) GCHK(G::fin_pseudo(gc, c.stream, k, c.ctl));
                     ++k;
                 }
                 if (int rc = poll(ctx)) return rc;
@@ -642,7 +643,7 @@ int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, 
     auto launch = [&]() -> hipError_t {
         if (which == 0) return G::cells(gc, c.stream, gc.U, gc.X, nullptr);
         if (g.dim == 3) return G::stage3(gc, c.stream, gc.U, gc.B, gc.S, gc.rk[0], which == 2, nullptr);
-        return G::iteration2(gc, c.stream, gc.B, gc.S, nullptr);
+        return G::iteration2(gc, c.stream, gc.B, gc.S, 0, false, nullptr);
     };
     GCHK(launch());
     GCHK(hipEventRecord(e0, c.stream));

@@ -240,6 +240,7 @@ struct StageLaunch {
     int foldp;              // modes 0, 1: cu, cv already hold -G p (launch_fold_gradp); p is not read
     double rk2;             // launch_stage_pair: the second stage's coefficient
     int pair;               // launch_stage_pair: 1 = stages 1-2, 2 = stages 3-4
+    int it, chained;        // launch_iteration: index in the step; 1: it also takes the norm of launch it - 1
     int expl;               // mode 1 with foldp: PSEUDO_TIMESTEPPING = 0's explicit update (rk = dt/1.5,
                             // base = stencil input = u^n; fluxTotal's domain ghosts 0, so wall faces
                             // take half the adjacent cell's flux)
@@ -253,6 +254,7 @@ bool stage_pair_fits(const Ctx &c);
 // one pseudo-iteration in one launch (k_iter_tile) from the base a.ub, a.vb into a.uo, a.vo
 bool iter_tile_wanted(const Ctx &c);
 hipError_t launch_iteration(const Ctx &c, const StageLaunch &a, int *nblocks);
+const double *iteration_partials(const Ctx &c, int it);  // the norm records of launch `it` of a step
 // cu, cv += -G p on the interior faces, once per FP64 step (p fixed over its pseudo-iterations)
 hipError_t launch_fold_gradp(const Ctx &c);
 // mixed (defect-correction) pseudo-iteration: see kernels_stage.hip
@@ -280,7 +282,8 @@ hipError_t launch_mixed_pair(const Ctx &c, const MixedPairLaunch &a, int *nblock
 bool mixed_pair_fits(const Ctx &c);
 // the pseudo-iteration norm and loop control (k_mixed_pair's records when the
 // step runs it); start_mg: also the Poisson phase's start (k_mg_start)
-hipError_t launch_fin_pseudo(const Ctx &c, int nblocks, int start_mg = 0);
+// (it: the launch's index in the step, where it was launch_iteration's)
+hipError_t launch_fin_pseudo(const Ctx &c, int nblocks, int start_mg = 0, int it = 0);
 // the norm of PSEUDO_TIMESTEPPING = 0's single update: ends the loop, countIter stays 0
 hipError_t launch_fin_explicit(const Ctx &c, int nblocks);
 hipError_t launch_ctl_reset_step(const Ctx &c);

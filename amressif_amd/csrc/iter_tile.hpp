@@ -14,7 +14,11 @@ struct IterTile {
     double *uo, *vo;        // u^{k+1}; must not alias u, v
     const double *lid;      // per-column velocity of the north side (kind 3), or null: inflow
     double *partials;       // records of `rec` doubles, the first two written: sum of the weighted change^2 of u and v
-    const Ctl *guard;       // null: unguarded
+    Ctl *ctl;               // null: unguarded
+    // records of the launch before, if its norm has not been taken yet: this launch then ends the loop
+    // itself where k_fin_pseudo would have (null: the control block is up to date)
+    const double *prev;
+    int it;                 // pseudo-iterations of the step before this launch
     int n, su, sv;          // cells per side, row strides of the x- and y-faces
     int rec;
     int copy_done;  // a launch past convergence copies u^k to the output (else it writes nothing)

@@ -816,15 +816,21 @@ int stage3_blocks(const Ctx &c)
     return c.s3_ntx * c.s3_nty * ((c.g.n + 1 + c.s3_zc - 1) / c.s3_zc);
 }
 
-hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, const Ctl *guard)
+// 2D: two sets of norm records in turn (a launch reads the one before's while it writes its own)
+static double *records2(const Ctx &c, int it) { return c.partials + (it & 1) * 3 * (int64_t)iter_tile_blocks(c.g.n); }
+
+hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, int it, bool chained,
+                      Ctl *ctl)
 {
     IterTile a{};
     const Geom &g = c.g;
     a.u = base[0]; a.v = base[1];
     a.cu = c.C[0]; a.cv = c.C[1];
     a.uo = out[0]; a.vo = out[1];
-    a.partials = c.partials;
-    a.guard = guard;
+    a.partials = records2(c, it);
+    a.prev = chained ? records2(c, it + 1) : nullptr;
+    a.it = it;
+    a.ctl = ctl;
     a.n = g.n;
     a.su = g.n + 1;
     a.sv = g.n;
@@ -879,10 +885,11 @@ hipError_t stage3(const Ctx &c, hipStream_t s, double *const *in, double *const 
     return hipGetLastError();
 }
 
-hipError_t fin_pseudo(const Ctx &c, hipStream_t s, Ctl *ctl)
+hipError_t fin_pseudo(const Ctx &c, hipStream_t s, int it, Ctl *ctl)
 {
     const int nrec = c.g.dim == 3 ? stage3_blocks(c) : iter_tile_blocks(c.g.n);
-    hipLaunchKernelGGL(k_gen_fin_pseudo, dim3(1), dim3(1024), 0, s, c.g, c.partials, nrec, ctl);
+    hipLaunchKernelGGL(k_gen_fin_pseudo, dim3(1), dim3(1024), 0, s, c.g, c.g.dim == 3 ? c.partials : records2(c, it), nrec,
+                       ctl);
     return hipGetLastError();
 }
 

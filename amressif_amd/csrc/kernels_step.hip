@@ -96,13 +96,14 @@ __global__ __launch_bounds__(1024) void k_fin_pseudo3(const double *partials, in
     }
 }
 
-hipError_t launch_fin_pseudo(const Ctx &c, int nblocks, int start_mg)
+hipError_t launch_fin_pseudo(const Ctx &c, int nblocks, int start_mg, int it)
 {
     if (c.mp_on)
         hipLaunchKernelGGL(k_fin_pseudo3, dim3(1), dim3(1024), 0, c.stream, c.partials, nblocks, c.ctl, c.g.n,
                            start_mg, c.g.dt);
     else
-        hipLaunchKernelGGL(k_fin_pseudo, dim3(1), dim3(1024), 0, c.stream, c.partials, nblocks, c.ctl, c.g.n);
+        hipLaunchKernelGGL(k_fin_pseudo, dim3(1), dim3(1024), 0, c.stream, iteration_partials(c, it), nblocks, c.ctl,
+                           c.g.n);
     return hipGetLastError();
 }
 

@@ -353,6 +353,42 @@ def test_one_launch_pseudo_iteration_matches_four_stage_launches(n, init, bc, li
     assert rel(p1 - p1.mean(), p4 - p4.mean()) < 1e-11
 
 
+@pytest.mark.parametrize("n", [40, 320])
+@pytest.mark.parametrize("end", ["cap", "diverged", "nonfinite"])
+def test_one_launch_pseudo_iteration_ends_the_loop_like_its_finalizer(n, end):
+    """A tile launch takes the norm of the launch before it and ends the loop
+    itself: at the iteration cap, past the divergence guard and on a norm that
+    is no number, inside a batch (the second and third step launch as many
+    pseudo-iterations as the step before needed), with the flags, counts and
+    norms of the separate finalizer."""
+    api = _api()
+
+    def run():
+        inp = api.cavity_inputs(n, 400.0, IterNum=3 if end == "cap" else 100, cfl=0.5,
+                                momentum_tolerance=1e-30 if end == "cap" else 1e-10)
+        r = api.Run.from_numpy(inp, W.initial_state(n, "seeded"))
+        st = [r.advance(2)]
+        if end != "cap":  # the third step's first norms end the loop within the batch
+            lid = np.zeros(n)
+            lid[n // 2] = 1e9 if end == "diverged" else np.inf
+            r.ctx.set_lid_profile(cuda(lid))
+            if end == "nonfinite":
+                with pytest.raises(api.AmressifError, match="non-finite pseudo-iteration norm at step 0"):
+                    r.advance(1)
+            else:
+                st.append(r.advance(1))
+        return [s for part in st for s in part]
+
+    s4 = _with_env({"AMRESSIF_STAGE_PAIR": "0"}, run)
+    s1 = _with_env({"AMRESSIF_ITER_TILE": "2"}, run)
+    print(f"n={n} {end}: {[(s['pseudo_iters'], s['flags'], s['norm_error']) for s in s1]}")
+    assert s1[-1]["flags"] == {"cap": api.FLAG_CAP, "diverged": api.FLAG_DIVERGED, "nonfinite": 0}[end]
+    for a, b in zip(s1, s4):
+        assert a["pseudo_iters"] == b["pseudo_iters"] and a["flags"] == b["flags"]
+        # the change of an iteration is a difference of O(1) velocities: exact to some eps of them
+        assert abs(a["norm_error"] - b["norm_error"]) <= 1e-9 * b["norm_error"] + 1e-15
+
+
 @pytest.mark.parametrize("n,rows,init,bc,lid", [
     (8, 4, "seeded", 0, False), (64, 4, "seeded", 0, False), (64, 5, "seeded", 1, False),
     (100, 16, "seeded", 2, True), (130, 7, "seeded", 0, False), (256, 16, "seeded", 3, False),
