@@ -217,8 +217,7 @@ int composite_solve(amressif_amr *A, int *iters, double *res_rel)
             for (int sweep = 0; sweep < 2; ++sweep)
                 for (int color = 0; color < 2; ++color)
                     ACHK(amr::amr_fine_gs(a, s, A->zcur, A->zcur + A->off1, A->vcur + A->off1, color, cc.ctl));
-            ACHK(amr::amr_cgm_apply(a, s, g));
-            ACHK(amr::amr_cgm_orthonormalise(a, s, g));
+            ACHK(amr::amr_cgm_arnoldi(a, s, g));
         }
         ACHK(amr::amr_cgm_edge(a, s, g));
         if (int rc2 = amr_poll(A->coarse)) return afail(A, rc2, amressif_last_error(A->coarse));
@@ -390,7 +389,7 @@ int amressif_amr_create(const amressif_inputs *in, int patch_jlo, void *hip_stre
     ACHK(hipHostMalloc((void **)&A->ctlF_host, sizeof(amr::Ctl), hipHostMallocDefault));
     const int nblk = amr::amr_flat_blocks(a);
     A->m = std::max(4, std::min(in->gmres_restart > 0 ? in->gmres_restart : 30, 60));
-    AALLOC(&A->part, (size_t)nblk * (A->m + 2));
+    AALLOC(&A->part, std::max((size_t)nblk * (A->m + 2), amr::cgm_partials_doubles(A->a, A->m)));
     AALLOC(&A->red, (size_t)A->m + 2);
     AALLOC(&A->coef, (size_t)A->m + 2);
     ACHK(hipHostMalloc((void **)&A->red_host, sizeof(double) * (A->m + 2), hipHostMallocDefault));

@@ -67,7 +67,8 @@ constexpr int kMaxPartials = 1 << 16;
 // Restarted FGMRES state (kernels_gmres.hip), device memory
 constexpr int kGmMax = 64;  // largest restart length
 struct GmState {
-    int j, total, pad0, pad1;  // Arnoldi step in the cycle, steps in the solve
+    int j, total;  // Arnoldi step in the cycle, steps in the solve
+    int jn, pad;   // two-level solve: j as the launch that writes j reads it
     double beta, target, scale;
     double gv[kGmMax + 1], cs[kGmMax], sn[kGmMax], y[kGmMax], c[kGmMax + 1];
     double H[(kGmMax + 1) * kGmMax];  // Hessenberg, row-major, reduced to R by Givens rotations
@@ -412,17 +413,14 @@ struct CgmBufs {
     double *x, *b;   // iterate and right-hand side
     double *vcur;    // the preconditioner's input (V_j normalised)
     double *zcur;    // and its output
-    double *part;    // flat blocks x (m + 2) partials
+    double *part;    // cgm_partials_doubles
     size_t vs, off1;
     int m;
 };
 hipError_t amr_cgm_begin(hipStream_t s, Ctl *ctl, GmState *st);
 hipError_t amr_cgm_edge(const AmrGeom &a, hipStream_t s, const CgmBufs &g);
-hipError_t amr_cgm_apply(const AmrGeom &a, hipStream_t s, const CgmBufs &g);
-hipError_t amr_cgm_orthonormalise(const AmrGeom &a, hipStream_t s, const CgmBufs &g);
-// the Arnoldi finalizers of kernels_gmres.hip on an nblk x (m + 2) partials layout
-hipError_t launch_gm_fin_dots_raw(hipStream_t s, double *part, int nblk, int m, GmState *st, Ctl *ctl, int pass);
-hipError_t launch_gm_fin_arnoldi_raw(hipStream_t s, double *part, int nblk, int m, GmState *st, Ctl *ctl);
+size_t cgm_partials_doubles(const AmrGeom &a, int m);
+hipError_t amr_cgm_arnoldi(const AmrGeom &a, hipStream_t s, const CgmBufs &g);
 hipError_t amr_rhs(const AmrGeom &a, hipStream_t s, double dt, const double *u0, const double *v0, const double *u1,
                    const double *v1, double *b0, double *b1, double *partials);
 hipError_t amr_project(const AmrGeom &a, hipStream_t s, double dt, const double *phi0, const double *phi1, double *u0,

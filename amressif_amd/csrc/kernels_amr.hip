@@ -410,10 +410,14 @@ __device__ double fine_L(const AmrGeom &a, const double *x0, const double *x1, i
 __device__ __forceinline__ bool flat_cell(const AmrGeom &a, long long k, int &lev, int &i, int &j)
 {
     const long long nc = (long long)a.n0 * a.jc0;
-    if (k < nc) { lev = 0; i = (int)(k % a.n0); j = (int)(k / a.n0); return true; }
-    k -= nc;
-    if (k < (long long)a.nx * a.ny) { lev = 1; i = (int)(k % a.nx); j = (int)(k / a.nx); return true; }
-    return false;
+    lev = k >= nc;
+    if (lev) k -= nc;
+    const int w = lev ? a.nx : a.n0;
+    if (k >= (lev ? (long long)a.nx * a.ny : nc)) return false;
+    // (a 64-bit division is some hundred instructions)
+    j = k >> 32 ? (int)(k / w) : (int)((unsigned)k / (unsigned)w);
+    i = (int)(k - (long long)w * j);
+    return true;
 }
 
 // y = b - L_c x (or y = L_c x with b null); partials: ||y||inf, ||y||_2^2
@@ -925,58 +929,315 @@ __global__ __launch_bounds__(256) void k_cgm_load(AmrGeom a, double *V, size_t v
     vcur[q] = x;
 }
 
-// Z_j = zcur; V_{j+1} = L_c zcur
-__global__ __launch_bounds__(256) void k_cgm_apply(AmrGeom a, const double *zcur, double *Z, double *V, size_t vs,
-                                                   const GmState *st, const Ctl *ctl, size_t off1)
+// One Arnoldi step (z = zcur already holds M V_j) in four launches over chunks of
+// composite cells, one chunk per workgroup: w = L_c z with the partials of <w, V_t>;
+// the classical Gram-Schmidt update, with the partials of the second pass over the
+// updated w; the second update, with the partials of ||w||^2; the Givens rotations and
+// the next V_j.  Each launch reduces the partials of the one before in every
+// workgroup, in the same order, instead of a one-workgroup launch between them.
+// Latency bound at the sizes of a two-level step (each vector is a few MB and stays
+// in the cache): nine launches, 77 us a step before, now 37 (512^2 and a 1024 x 256
+// patch, restart 30, 4 steps a cycle).
+constexpr int kCgmCells = 4;             // cells per thread and batch (their loads are in flight together)
+constexpr int kCgmMaxChunks = 1024;      // workgroups: 4 waves per SIMD; more cells lengthen the chunks
+constexpr int kCgmGroup = 4;             // V_t of one pass over the cells
+
+struct Cgm {
+    AmrGeom a;
+    double *V, *Z;
+    const double *zcur;
+    double *vcur;
+    double *part;   // <w, V_t> of the first pass, of the second pass (m + 1 each), ||w||^2: nchunk each
+    size_t vs, off1;
+    GmState *st;
+    Ctl *ctl;
+    int m, nchunk;
+    long long chunk;  // cells per workgroup, a multiple of 256
+};
+
+__device__ __forceinline__ double cgm_wave_sum(double x)
 {
-    if (cgm_iter_skip(ctl)) return;
-    const long long k = blockIdx.x * 256LL + threadIdx.x;
-    int lev, i, j;
-    if (!flat_cell(a, k, lev, i, j)) return;
-    const size_t q = comp_index(a, lev, i, j, off1);
-    const int jj = st->j;
-    Z[(size_t)jj * vs + q] = zcur[q];
-    V[(size_t)(jj + 1) * vs + q] = lev == 0 ? coarse_L(a, zcur, zcur + off1, i, j) : fine_L(a, zcur, zcur + off1, i, j);
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    return x;
 }
 
-// partials of <V_{j+1}, V_t>, t <= j, into slot t of each block's m + 2
-__global__ __launch_bounds__(256) void k_cgm_dots(AmrGeom a, const double *V, size_t vs, const GmState *st,
-                                                  const Ctl *ctl, size_t off1, double *partials, int m)
+// the batch of the chunk's cells from k0.  Off the chunk the index of a cell that
+// exists, so that every load of a batch can go out unconditionally (loads under a
+// condition of their own wait for each other: k_cgm_apply 15 us instead of 11).
+struct CgmBatch {
+    size_t q[kCgmCells];
+    bool ok[kCgmCells];
+    int lev[kCgmCells], i[kCgmCells], j[kCgmCells];
+};
+__device__ __forceinline__ CgmBatch cgm_batch(const Cgm &g, long long k0)
 {
-    __shared__ double sh[16];
-    if (cgm_iter_skip(ctl)) return;
-    const long long k = blockIdx.x * 256LL + threadIdx.x;
-    int lev, i, j;
-    const bool ok = flat_cell(a, k, lev, i, j);
-    const size_t q = ok ? comp_index(a, lev, i, j, off1) : 0;
-    const int jj = st->j;
-    const double wq = ok ? V[(size_t)(jj + 1) * vs + q] : 0.0;
-    for (int t = 0; t <= jj; ++t) {
-        double acc = ok ? wq * V[(size_t)t * vs + q] : 0.0;
-        acc = block_reduce<false>(acc, sh);
-        if (threadIdx.x == 0) partials[(size_t)blockIdx.x * (m + 2) + t] = acc;
+    const long long end = ((long long)blockIdx.x + 1) * g.chunk;
+    CgmBatch b;
+#pragma unroll
+    for (int c = 0; c < kCgmCells; ++c) {
+        const long long k = k0 + 256 * c + threadIdx.x;
+        b.ok[c] = flat_cell(g.a, k, b.lev[c], b.i[c], b.j[c]) && k < end;
+        if (!b.ok[c]) b.lev[c] = 1, b.i[c] = b.j[c] = 0;
+        b.q[c] = comp_index(g.a, b.lev[c], b.i[c], b.j[c], g.off1);
+    }
+    return b;
+}
+
+// L_c x over a batch: coarse_L and fine_L with the loads of all cells first (a wall's
+// neighbour is the cell itself: no flux), then the coarse-fine interface's gradients
+__device__ __forceinline__ void cgm_apply_batch(const Cgm &g, const CgmBatch &b, const double *x,
+                                                double (&c0)[kCgmCells], double (&y)[kCgmCells])
+{
+    double w[kCgmCells], e[kCgmCells], s[kCgmCells], n[kCgmCells];
+#pragma unroll
+    for (int c = 0; c < kCgmCells; ++c) {
+        const int nx = b.lev[c] ? g.a.nx : g.a.n0, ny = b.lev[c] ? g.a.ny : g.a.jc0, P = b.lev[c] ? g.a.P1 : g.a.P0;
+        const double *xq = x + b.q[c];
+        c0[c] = xq[0];
+        w[c] = xq[b.i[c] > 0 ? -1 : 0];
+        e[c] = xq[b.i[c] < nx - 1 ? 1 : 0];
+        s[c] = xq[b.j[c] > 0 ? -P : 0];
+        n[c] = xq[b.j[c] < ny - 1 ? P : 0];
+    }
+#pragma unroll
+    for (int c = 0; c < kCgmCells; ++c) {
+        const double ih = 1.0 / (b.lev[c] ? g.a.h1 : g.a.h0);
+        const double fw = (c0[c] - w[c]) * ih, fe = (e[c] - c0[c]) * ih;
+        double fs = (c0[c] - s[c]) * ih, fn = (n[c] - c0[c]) * ih;
+        const double *x1 = x + g.off1;
+        if (b.lev[c] ? b.j[c] == 0 : b.j[c] == g.a.jc0 - 1) {
+            if (b.lev[c]) fs = (c0[c] - cf_ghost(g.a, x, x1, b.i[c])) * ih;
+            else {  // mean of the two fine interface gradients above
+                const int f0 = 2 * b.i[c];
+                const double g0 = (x1[f0] - cf_ghost(g.a, x, x1, f0)) / g.a.h1;
+                const double g1 = (x1[f0 + 1] - cf_ghost(g.a, x, x1, f0 + 1)) / g.a.h1;
+                fn = 0.5 * (g0 + g1);
+            }
+        }
+        y[c] = (fe - fw) * ih + (fn - fs) * ih;
     }
 }
 
-// V_{j+1} -= sum_t c_t V_t; partial ||V_{j+1}||_2^2 into slot m + 1
-__global__ __launch_bounds__(256) void k_cgm_orth(AmrGeom a, double *V, size_t vs, const GmState *st, const Ctl *ctl,
-                                                  size_t off1, double *partials, int m)
+// acc[u] += w V_{t0 + u} of the batch; a group that reaches past V_jj repeats V_jj,
+// and those sums are not used
+__device__ __forceinline__ void cgm_dot_group(const Cgm &g, int t0, int jj, const CgmBatch &b,
+                                              const double (&w)[kCgmCells], double (&acc)[kCgmGroup])
 {
-    __shared__ double sh[16];
-    if (cgm_iter_skip(ctl)) return;
-    const long long k = blockIdx.x * 256LL + threadIdx.x;
-    int lev, i, j;
-    double s2 = 0.0;
-    if (flat_cell(a, k, lev, i, j)) {
-        const size_t q = comp_index(a, lev, i, j, off1);
-        const int jj = st->j;
-        double w = V[(size_t)(jj + 1) * vs + q];
-        for (int t = 0; t <= jj; ++t) w -= st->c[t] * V[(size_t)t * vs + q];
-        V[(size_t)(jj + 1) * vs + q] = w;
-        s2 = w * w;
+    double v[kCgmGroup][kCgmCells];
+#pragma unroll
+    for (int u = 0; u < kCgmGroup; ++u)
+#pragma unroll
+        for (int c = 0; c < kCgmCells; ++c) v[u][c] = g.V[(size_t)min(t0 + u, jj) * g.vs + b.q[c]];
+#pragma unroll
+    for (int u = 0; u < kCgmGroup; ++u)
+#pragma unroll
+        for (int c = 0; c < kCgmCells; ++c) acc[u] += w[c] * v[u][c];  // (w = 0 off the chunk)
+}
+
+// the workgroup's sums of a group into the partials of slots t0.. (p: the pass's)
+__device__ __forceinline__ void cgm_put_group(const Cgm &g, double *p, int t0, int jj, double (&acc)[kCgmGroup],
+                                              double (&sh)[4][kCgmGroup])
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int u = 0; u < kCgmGroup; ++u) acc[u] = cgm_wave_sum(acc[u]);
+    __syncthreads();  // sh's readers of the group before
+    if (lane == 0)
+#pragma unroll
+        for (int u = 0; u < kCgmGroup; ++u) sh[wid][u] = acc[u];
+    __syncthreads();
+    const int u = threadIdx.x;
+    if (u < kCgmGroup && t0 + u <= jj)
+        p[(size_t)(t0 + u) * g.nchunk + blockIdx.x] = sh[0][u] + sh[1][u] + sh[2][u] + sh[3][u];
+}
+
+// sums over the chunks of slots 0..jj (one wave per slot) into shC, zero past jj to
+// the end of its group
+__device__ __forceinline__ void cgm_get(const Cgm &g, const double *p, int jj, double *shC)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    for (int t = wid; t < (jj / kCgmGroup + 1) * kCgmGroup; t += 4) {
+        double s = 0.0;
+        if (t <= jj)
+            for (int b0 = 0; b0 < g.nchunk; b0 += 512) {  // eight loads in flight
+                double v[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) v[r] = p[(size_t)t * g.nchunk + min(b0 + 64 * r + lane, g.nchunk - 1)];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) s += b0 + 64 * r + lane < g.nchunk ? v[r] : 0.0;
+            }
+        s = cgm_wave_sum(s);
+        if (lane == 0) shC[t] = s;
     }
-    s2 = block_reduce<false>(s2, sh);
-    if (threadIdx.x == 0) partials[(size_t)blockIdx.x * (m + 2) + m + 1] = s2;
+    __syncthreads();
+}
+
+// Z_j = zcur, w = L_c zcur into V_{j+1}
+__global__ __launch_bounds__(256) void k_cgm_apply(Cgm g)
+{
+    __shared__ double sh[4][kCgmGroup];
+    if (cgm_iter_skip(g.ctl)) return;
+    const int jj = g.st->j;
+    double *z = g.Z + (size_t)jj * g.vs, *w = g.V + (size_t)(jj + 1) * g.vs;
+    const long long k0 = blockIdx.x * g.chunk;
+    if (blockIdx.x == 0 && threadIdx.x == 0) g.st->jn = jj;
+    for (int t0 = 0; t0 <= jj; t0 += kCgmGroup) {
+        double acc[kCgmGroup] = {};
+        for (long long kb = k0; kb < k0 + g.chunk; kb += 256 * kCgmCells) {
+            const CgmBatch b = cgm_batch(g, kb);
+            double x[kCgmCells];
+            if (t0 == 0) {
+                double c0[kCgmCells];
+                cgm_apply_batch(g, b, g.zcur, c0, x);
+#pragma unroll
+                for (int c = 0; c < kCgmCells; ++c)
+                    if (b.ok[c]) {
+                        z[b.q[c]] = c0[c];
+                        w[b.q[c]] = x[c];
+                    }
+            } else {
+#pragma unroll
+                for (int c = 0; c < kCgmCells; ++c) x[c] = w[b.q[c]];
+            }
+#pragma unroll
+            for (int c = 0; c < kCgmCells; ++c) x[c] = b.ok[c] ? x[c] : 0.0;
+            cgm_dot_group(g, t0, jj, b, x, acc);
+        }
+        cgm_put_group(g, g.part, t0, jj, acc, sh);
+    }
+}
+
+// w -= sum_t c_t V_t with c from the partials of pass PASS (0, 1); then pass 0: the
+// partials of pass 1, pass 1: the partials of ||w||^2
+template <int PASS>
+__global__ __launch_bounds__(256) void k_cgm_orth(Cgm g)
+{
+    __shared__ double sh[4][kCgmGroup], shC[kGmMax + kCgmGroup];
+    if (cgm_iter_skip(g.ctl)) return;
+    const int jj = g.st->j;
+    double *w = g.V + (size_t)(jj + 1) * g.vs;
+    const size_t set = (size_t)(g.m + 1) * g.nchunk;
+    cgm_get(g, g.part + PASS * set, jj, shC);
+    if (blockIdx.x == 0)
+        for (int t = threadIdx.x; t <= jj; t += 256) {  // H(:, j): the two passes' sum
+            double &h = g.st->H[t * kGmMax + jj];
+            h = PASS ? h + shC[t] : shC[t];
+        }
+    const long long k0 = blockIdx.x * g.chunk;
+    for (int t0 = 0; t0 <= (PASS ? 0 : jj); t0 += kCgmGroup) {
+        double acc[kCgmGroup] = {};
+        for (long long kb = k0; kb < k0 + g.chunk; kb += 256 * kCgmCells) {
+            const CgmBatch b = cgm_batch(g, kb);
+            double x[kCgmCells];
+#pragma unroll
+            for (int c = 0; c < kCgmCells; ++c) x[c] = w[b.q[c]];
+            if (t0 == 0) {
+                for (int t = 0; t <= jj; t += kCgmGroup) {
+                    double v[kCgmGroup][kCgmCells];
+#pragma unroll
+                    for (int u = 0; u < kCgmGroup; ++u)
+#pragma unroll
+                        for (int c = 0; c < kCgmCells; ++c) v[u][c] = g.V[(size_t)min(t + u, jj) * g.vs + b.q[c]];
+#pragma unroll
+                    for (int u = 0; u < kCgmGroup; ++u)
+#pragma unroll
+                        for (int c = 0; c < kCgmCells; ++c) x[c] -= shC[t + u] * v[u][c];
+                }
+#pragma unroll
+                for (int c = 0; c < kCgmCells; ++c)
+                    if (b.ok[c]) w[b.q[c]] = x[c];
+            }
+#pragma unroll
+            for (int c = 0; c < kCgmCells; ++c) {
+                x[c] = b.ok[c] ? x[c] : 0.0;
+                if (PASS) acc[0] += x[c] * x[c];
+            }
+            if (!PASS) cgm_dot_group(g, t0, jj, b, x, acc);
+        }
+        if (PASS) cgm_put_group(g, g.part + 2 * set, 0, 0, acc, sh);
+        else cgm_put_group(g, g.part + set, t0, jj, acc, sh);
+    }
+}
+
+// h_{j+1,j} = ||w||, the Givens rotations and the residual estimate (the first
+// workgroup's first wave: lane t holds row t of the column); V_{j+1} normalised, into
+// vcur too.  The stop test of this launch may be seen by later workgroups, which then
+// leave V_{j+1} as it is: the cycle has ended and does not use it.
+__global__ __launch_bounds__(256) void k_cgm_next(Cgm g)
+{
+    __shared__ double shC[kGmMax + kCgmGroup];
+    __shared__ int shSkip;
+    if (threadIdx.x == 0)
+        shSkip = __hip_atomic_load(&g.ctl->mg_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) |
+                 __hip_atomic_load(&g.ctl->gm_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    cgm_get(g, g.part + 2 * (size_t)(g.m + 1) * g.nchunk, 0, shC);  // (ends with a barrier)
+    if (shSkip) return;
+    const int jj = g.st->jn;
+    const double hn = sqrt(shC[0]);
+    const double sc = hn > 0.0 ? 1.0 / hn : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        GmState *st = g.st;
+        const int t = threadIdx.x;
+        double h = t <= jj ? st->H[t * kGmMax + jj] : 0.0;
+        const double csl = t < jj ? st->cs[t] : 1.0, snl = t < jj ? st->sn[t] : 0.0, gj = st->gv[jj];
+        double a = __shfl(h, 0, 64);
+        for (int v = 0; v < jj; ++v) {  // earlier rotations on column jj
+            const double b = __shfl(h, v + 1, 64), c = __shfl(csl, v, 64), s = __shfl(snl, v, 64);
+            if (t == v) h = c * a + s * b;
+            a = -s * a + c * b;
+        }
+        const double rr = sqrt(a * a + hn * hn);
+        const double cs = rr > 0.0 ? a / rr : 1.0, sn = rr > 0.0 ? hn / rr : 0.0;
+        if (t == jj) h = rr;
+        if (t <= jj) st->H[t * kGmMax + jj] = h;
+        if (t == 0) {
+            Ctl *ctl = g.ctl;
+            st->cs[jj] = cs;
+            st->sn[jj] = sn;
+            st->gv[jj + 1] = -sn * gj;
+            st->gv[jj] = cs * gj;
+            st->j = jj + 1;
+            st->total += 1;
+            const int it = ctl->mg_iters + 1;
+            ctl->mg_iters = it;
+            const double est = fabs(sn * gj);
+            const bool nan = !(est == est);
+            if (nan) ctl->flags |= AMRESSIF_FLAG_NONFINITE;
+            if (est <= st->target || hn == 0.0 || jj + 1 >= g.m || it >= ctl->mg_max_iter) ctl->gm_stop = 1;
+            if (nan) ctl->mg_done = 1;
+        }
+    }
+    double *w = g.V + (size_t)(jj + 1) * g.vs;
+    const long long k0 = blockIdx.x * g.chunk;
+    for (long long kb = k0; kb < k0 + g.chunk; kb += 256 * kCgmCells) {
+        const CgmBatch b = cgm_batch(g, kb);
+        double x[kCgmCells];
+#pragma unroll
+        for (int c = 0; c < kCgmCells; ++c) x[c] = w[b.q[c]] * sc;
+#pragma unroll
+        for (int c = 0; c < kCgmCells; ++c)
+            if (b.ok[c]) {
+                w[b.q[c]] = x[c];
+                g.vcur[b.q[c]] = x[c];
+            }
+    }
+}
+
+// chunks of whole batches, as many as fit
+static void cgm_chunks(const AmrGeom &a, int *nchunk, long long *chunk)
+{
+    const long long batch = 256 * kCgmCells, cells = (long long)a.n0 * a.jc0 + (long long)a.nx * a.ny;
+    const long long batches = (cells + batch - 1) / batch;
+    const long long per = (batches + kCgmMaxChunks - 1) / kCgmMaxChunks;
+    *chunk = per * batch;
+    *nchunk = (int)((batches + per - 1) / per);
+}
+size_t cgm_partials_doubles(const AmrGeom &a, int m)
+{
+    int nchunk;
+    long long chunk;
+    cgm_chunks(a, &nchunk, &chunk);
+    return (size_t)nchunk * (2 * (m + 1) + 1);
 }
 
 hipError_t amr_cgm_begin(hipStream_t s, Ctl *ctl, GmState *st)
@@ -999,28 +1260,25 @@ hipError_t amr_cgm_edge(const AmrGeom &a, hipStream_t s, const CgmBufs &g)
     return hipGetLastError();
 }
 
-hipError_t amr_cgm_apply(const AmrGeom &a, hipStream_t s, const CgmBufs &g)
+hipError_t amr_cgm_arnoldi(const AmrGeom &a, hipStream_t s, const CgmBufs &b)
 {
-    hipLaunchKernelGGL(k_cgm_apply, dim3(flat_blocks(a)), dim3(256), 0, s, a, (const double *)g.zcur, g.Z, g.V, g.vs,
-                       (const GmState *)g.st, (const Ctl *)g.ctl, g.off1);
-    return hipGetLastError();
-}
-
-// classical Gram-Schmidt twice, then ||w||, the Givens rotations and the
-// stopping estimate; then the next V_j is normalised into vcur
-hipError_t amr_cgm_orthonormalise(const AmrGeom &a, hipStream_t s, const CgmBufs &g)
-{
-    const int nb = flat_blocks(a);
-    for (int pass = 0; pass < 2; ++pass) {
-        hipLaunchKernelGGL(k_cgm_dots, dim3(nb), dim3(256), 0, s, a, (const double *)g.V, g.vs, (const GmState *)g.st,
-                           (const Ctl *)g.ctl, g.off1, g.part, g.m);
-        if (hipError_t e = launch_gm_fin_dots_raw(s, g.part, nb, g.m, g.st, g.ctl, pass)) return e;
-        hipLaunchKernelGGL(k_cgm_orth, dim3(nb), dim3(256), 0, s, a, g.V, g.vs, (const GmState *)g.st,
-                           (const Ctl *)g.ctl, g.off1, g.part, g.m);
-    }
-    if (hipError_t e = launch_gm_fin_arnoldi_raw(s, g.part, nb, g.m, g.st, g.ctl)) return e;
-    hipLaunchKernelGGL(k_cgm_load, dim3(nb), dim3(256), 0, s, a, g.V, g.vs, g.vcur, (const GmState *)g.st,
-                       (const Ctl *)g.ctl, g.off1);
+    Cgm g{};
+    g.a = a;
+    g.V = b.V;
+    g.Z = b.Z;
+    g.zcur = b.zcur;
+    g.vcur = b.vcur;
+    g.part = b.part;
+    g.vs = b.vs;
+    g.off1 = b.off1;
+    g.st = b.st;
+    g.ctl = b.ctl;
+    g.m = b.m;
+    cgm_chunks(a, &g.nchunk, &g.chunk);
+    hipLaunchKernelGGL(k_cgm_apply, dim3(g.nchunk), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_cgm_orth<0>, dim3(g.nchunk), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_cgm_orth<1>, dim3(g.nchunk), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_cgm_next, dim3(g.nchunk), dim3(256), 0, s, g);
     return hipGetLastError();
 }
 hipError_t amr_rhs(const AmrGeom &a, hipStream_t s, double dt, const double *u0, const double *v0, const double *u1,
