@@ -183,9 +183,7 @@ int precondition(amressif_amr *A, double *v, double *z)
     ACHK(amr::amr_restrict(a, s, v, v + A->off1, rc, A->mixed));
     ACHK(amr::launch_mg_start(cc));
     ACHK(amr::launch_vcycle(cc, A->mixed));
-    ACHK(amr::amr_prolong(a, s, e, z, z + A->off1, A->mixed));
-    for (int sweep = 0; sweep < 2; ++sweep)
-        for (int color = 0; color < 2; ++color) ACHK(amr::amr_fine_gs(a, s, z, z + A->off1, v + A->off1, color));
+    ACHK(amr::amr_prolong_gs(a, s, e, z, z + A->off1, v + A->off1, A->mixed));
     return 0;
 }
 
@@ -213,10 +211,7 @@ int composite_solve(amressif_amr *A, int *iters, double *res_rel)
             // red-black Gauss-Seidel sweeps on the patch
             ACHK(amr::amr_restrict(a, s, A->vcur, A->vcur + A->off1, rc, A->mixed, cc.ctl));
             ACHK(amr::launch_vcycle(cc, A->mixed));
-            ACHK(amr::amr_prolong(a, s, e, A->zcur, A->zcur + A->off1, A->mixed, cc.ctl));
-            for (int sweep = 0; sweep < 2; ++sweep)
-                for (int color = 0; color < 2; ++color)
-                    ACHK(amr::amr_fine_gs(a, s, A->zcur, A->zcur + A->off1, A->vcur + A->off1, color, cc.ctl));
+            ACHK(amr::amr_prolong_gs(a, s, e, A->zcur, A->zcur + A->off1, A->vcur + A->off1, A->mixed, cc.ctl));
             ACHK(amr::amr_cgm_arnoldi(a, s, g));
         }
         ACHK(amr::amr_cgm_edge(a, s, g));

@@ -401,10 +401,8 @@ hipError_t amr_shift(const AmrGeom &a, hipStream_t s, double *x0, double *x1, co
 // does nothing once its Arnoldi cycle or solve has ended)
 hipError_t amr_restrict(const AmrGeom &a, hipStream_t s, const double *r0, const double *r1, void *rc, int mixed,
                         const Ctl *guard = nullptr);
-hipError_t amr_prolong(const AmrGeom &a, hipStream_t s, const void *e, double *z0, double *z1, int mixed,
-                       const Ctl *guard = nullptr);
-hipError_t amr_fine_gs(const AmrGeom &a, hipStream_t s, const double *z0, double *z1, const double *r1, int color,
-                       const Ctl *guard = nullptr);
+hipError_t amr_prolong_gs(const AmrGeom &a, hipStream_t s, const void *e, double *z0, double *z1, const double *r1,
+                          int mixed, const Ctl *guard = nullptr);
 // device composite FGMRES (kernels_amr.hip): vectors [coarse | fine] of stride vs
 struct CgmBufs {
     Ctl *ctl;        // control: mg_done ends the solve, gm_stop the cycle

@@ -529,42 +529,77 @@ __global__ __launch_bounds__(256) void k_amr_restrict(AmrGeom a, const double *r
     rc[i + (size_t)a.P0 * j] = (T)v;
 }
 
-// coarse correction onto the composite vector: z0 = e, z1 = e of the covering
-// coarse cell
+// The coarse correction onto the composite vector (z0 = e, z1 = e of the covering
+// coarse cell), then two red-black Gauss-Seidel sweeps of L_1 z1 = r1 on the fine
+// patch (coarse values fixed in the C/F ghost), in one launch: a workgroup takes 56 x
+// 24 patch cells and a ring of four around them into LDS, and each of the four half
+// sweeps uses up one ring, so the values are those of the sweeps over the whole patch.
+// The workgroups past the tiles copy the coarse cells.  Launch bound: five launches, 20 us
+// before, now 10 (a 1024 x 256 patch).
+constexpr int kPgW = 64, kPgH = 32, kPgHalo = 4;  // the tile with its ring: one wave per row, 4 waves
+constexpr int kPgTx = kPgW - 2 * kPgHalo, kPgTy = kPgH - 2 * kPgHalo;
 template <class T>
-__global__ __launch_bounds__(256) void k_amr_prolong(AmrGeom a, const T *e, double *z0, double *z1, const Ctl *guard)
+__global__ __launch_bounds__(256) void k_amr_prolong_gs(AmrGeom a, const T *e, double *z0, double *z1, const double *r1,
+                                                        int ntx, int ntile, const Ctl *guard)
 {
+    __shared__ double z[kPgH][kPgW];
     if (cgm_iter_skip(guard)) return;
-    const long long k = blockIdx.x * 256LL + threadIdx.x;
-    int lev, i, j;
-    if (!flat_cell(a, k, lev, i, j)) return;
-    if (lev == 0) z0[i + (size_t)a.P0 * j] = (double)e[i + (size_t)a.P0 * j];
-    else z1[i + (size_t)a.P1 * j] = (double)e[(i >> 1) + (size_t)a.P0 * (a.jc0 + (j >> 1))];
-}
-
-// one red or black Gauss-Seidel half-sweep of L_1 z1 = r1 on the fine patch
-// (coarse values z0 fixed in the C/F ghost)
-__global__ __launch_bounds__(256) void k_amr_fine_gs(AmrGeom a, const double *z0, double *z1, const double *r1,
-                                                     int color, const Ctl *guard)
-{
-    if (cgm_iter_skip(guard)) return;
-    const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (i >= a.nx || j >= a.ny || ((i + j) & 1) != color) return;
-    const int P = a.P1;
-    const size_t k = i + (size_t)P * j;
-    const double ih2 = 1.0 / (a.h1 * a.h1);
-    double off = 0.0, diag = 0.0;
-    if (i > 0) { off += z1[k - 1]; diag += 1.0; }
-    if (i < a.nx - 1) { off += z1[k + 1]; diag += 1.0; }
-    if (j < a.ny - 1) { off += z1[k + P]; diag += 1.0; }
-    if (j > 0) { off += z1[k - P]; diag += 1.0; }
-    else {  // ghost = 8/15 pc + 2/3 z(i,0) - 1/5 z(i,1): fold its z(i,0) part into the diagonal
-        auto f = [&](int ic, int jc) { return z0[ic + (size_t)a.P0 * jc]; };
-        const double pc = tangential(f, a.n0, i, a.jc0 - 1);
-        off += (8.0 / 15.0) * pc - 0.2 * z1[k + P];
-        diag += 1.0 - 2.0 / 3.0;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if ((int)blockIdx.x >= ntile) {
+        const unsigned nc = (unsigned)a.n0 * a.jc0, kb = (blockIdx.x - ntile) * 1024u + threadIdx.x;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const unsigned k = min(kb + 256u * c, nc - 1);
+            const size_t q = k % (unsigned)a.n0 + (size_t)a.P0 * (k / (unsigned)a.n0);
+            z0[q] = (double)e[q];
+        }
+        return;
     }
-    z1[k] = (off - r1[k] / ih2) / diag;
+    const int P = a.P1;
+    const int i = ((int)blockIdx.x % ntx) * kPgTx - kPgHalo + lane, jt = ((int)blockIdx.x / ntx) * kPgTy - kPgHalo;
+    const bool in = i >= 0 && i < a.nx;
+    const double ih2 = 1.0 / (a.h1 * a.h1);
+    double r[kPgH / 8][2];  // rows 2 (wid + 4 p) and the next
+#pragma unroll
+    for (int p = 0; p < kPgH / 8; ++p)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int row = 2 * (wid + 4 * p) + b, j = jt + row;
+            const int ic = min(max(i, 0), a.nx - 1), jc = min(max(j, 0), a.ny - 1);
+            z[row][lane] = (double)e[(ic >> 1) + (size_t)a.P0 * (a.jc0 + (jc >> 1))];
+            r[p][b] = r1[ic + (size_t)P * jc] / ih2;
+        }
+    double pc = 0.0;  // the ghost's tangential part, below the patch's first row
+    if (jt < 0 && in)
+        pc = tangential([&](int c, int jc) { return (double)e[c + (size_t)a.P0 * jc]; }, a.n0, i, a.jc0 - 1);
+    const int cw = i > 0 ? max(lane - 1, 0) : lane, ce = i < a.nx - 1 ? min(lane + 1, 63) : lane;
+    const double fw = i > 0 ? 1.0 : 0.0, fe = i < a.nx - 1 ? 1.0 : 0.0;
+    // (the tile's edge columns and rows have no outer neighbour to use: they keep their value)
+    const bool upd = in && (lane > 0 || i == 0) && (lane < 63 || i == a.nx - 1);
+    for (int h = 0; h < 4; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < kPgH / 8; ++p) {
+            // the cell of this column and colour in the row pair
+            const int b = (i + jt + h) & 1, row = 2 * (wid + 4 * p) + b, j = jt + row;
+            if (!upd || j < 0 || j >= a.ny || (row == 0 && j > 0) || (row == kPgH - 1 && j < a.ny - 1)) continue;
+            const double rr = b ? r[p][1] : r[p][0];
+            double off = 0.0, diag = fw + fe;
+            if (i > 0) off += z[row][cw];
+            if (i < a.nx - 1) off += z[row][ce];
+            if (j < a.ny - 1) { off += z[row + 1][lane]; diag += 1.0; }
+            if (j > 0) { off += z[row - 1][lane]; diag += 1.0; }
+            else {  // ghost = 8/15 pc + 2/3 z(i,0) - 1/5 z(i,1): fold its z(i,0) part into the diagonal
+                off += (8.0 / 15.0) * pc - 0.2 * z[row + 1][lane];
+                diag += 1.0 - 2.0 / 3.0;
+            }
+            z[row][lane] = diag == 4.0 ? (off - rr) * 0.25 : (off - rr) / diag;
+        }
+    }
+    __syncthreads();
+    if (lane < kPgHalo || lane >= kPgHalo + kPgTx || !in) return;
+    for (int row = kPgHalo + wid; row < kPgHalo + kPgTy && jt + row < a.ny; row += 4)
+        z1[i + (size_t)P * (jt + row)] = z[row][lane];
 }
 
 // ------------------------------------------------------------ projection
@@ -779,21 +814,17 @@ hipError_t amr_restrict(const AmrGeom &a, hipStream_t s, const double *r0, const
         hipLaunchKernelGGL(k_amr_restrict<double>, g2(a.n0, a.n0), dim3(256), 0, s, a, r0, r1, (double *)rc, guard);
     return hipGetLastError();
 }
-hipError_t amr_prolong(const AmrGeom &a, hipStream_t s, const void *e, double *z0, double *z1, int mixed,
-                       const Ctl *guard)
+hipError_t amr_prolong_gs(const AmrGeom &a, hipStream_t s, const void *e, double *z0, double *z1, const double *r1,
+                          int mixed, const Ctl *guard)
 {
+    const int ntx = (a.nx + kPgTx - 1) / kPgTx, ntile = ntx * ((a.ny + kPgTy - 1) / kPgTy);
+    const dim3 grid(ntile + (int)(((long long)a.n0 * a.jc0 + 1023) / 1024));
     if (mixed)
-        hipLaunchKernelGGL(k_amr_prolong<float>, dim3(flat_blocks(a)), dim3(256), 0, s, a, (const float *)e, z0, z1,
+        hipLaunchKernelGGL(k_amr_prolong_gs<float>, grid, dim3(256), 0, s, a, (const float *)e, z0, z1, r1, ntx, ntile,
                            guard);
     else
-        hipLaunchKernelGGL(k_amr_prolong<double>, dim3(flat_blocks(a)), dim3(256), 0, s, a, (const double *)e, z0, z1,
-                           guard);
-    return hipGetLastError();
-}
-hipError_t amr_fine_gs(const AmrGeom &a, hipStream_t s, const double *z0, double *z1, const double *r1, int color,
-                       const Ctl *guard)
-{
-    hipLaunchKernelGGL(k_amr_fine_gs, g2(a.nx, a.ny), dim3(256), 0, s, a, z0, z1, r1, color, guard);
+        hipLaunchKernelGGL(k_amr_prolong_gs<double>, grid, dim3(256), 0, s, a, (const double *)e, z0, z1, r1, ntx,
+                           ntile, guard);
     return hipGetLastError();
 }
 

@@ -120,6 +120,24 @@ def test_patch_bounds_are_checked():
         _two_level(32, 1, 100.0)
 
 
+@pytest.mark.parametrize("n0,jc0,restart,prec,iters", [
+    (8, 2, 4, 0, (13, 10, 10)), (28, 26, 5, 0, (7, 11, 11)), (30, 4, 9, 0, (8, 8, 8)), (46, 31, 30, 1, (8, 8, 8)),
+    (52, 28, 6, 0, (8, 8, 8)), (700, 350, 5, 1, (12, 12, 11))])
+def test_composite_solve_at_tile_and_chunk_edges(n0, jc0, restart, prec, iters):
+    """The patch sweeps in LDS tiles (56 x 24 cells) and the Arnoldi step in
+    chunks of 1024 cells: patches below, at and past a tile, one and two batches
+    per chunk (more than 1024 x 1024 cells), restarts that end a cycle within a
+    group of four Arnoldi vectors, at one and past one.  iters: what the solve
+    takes with the sweeps as launches over the whole patch; one more where the
+    order of the sums moves the last residual over the tolerance."""
+    api = _api()
+    tl = _two_level(n0, jc0, 2000.0, precision=prec, gmres_restart=restart)
+    for s, want in zip(tl.advance(3), iters):
+        assert s["flags"] == 0, s
+        assert s["poisson_res"] <= 1e-10 and s["poisson_iters"] <= want + 1, (s, want)
+        assert s["div_new"] <= 1e-9 * s["div_star"] + 1e-10, s
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 def test_device_composite_fgmres_matches_the_host_driven_one(prec):
     """The composite FGMRES with its Arnoldi process on the device (one host
