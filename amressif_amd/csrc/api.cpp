@@ -971,23 +971,31 @@ int amressif_create(const amressif_inputs *in, void *hip_stream, amressif_ctx **
                                                       "with an odd m > 2048)");
             const int bx = B.nx, by = B.ny;
             const double pi = 3.14159265358979323846;
-            std::vector<double> tab((size_t)bx * bx + (size_t)by * by + (size_t)by * bx);
-            auto fill = [&](double *Cm, int m) {
+            c.big_strip = amr::bottom_strips(bx, by);
+            const int lx = c.big_strip ? (int)round_up(bx, 128) : bx, ly = c.big_strip ? (int)round_up(by, 128) : by;
+            // C_x, C_y and D+; strip-wise also C_x^T and C_y^T, all padded with zeros
+            std::vector<double> tab((c.big_strip ? 2 : 1) * ((size_t)lx * lx + (size_t)ly * ly) + (size_t)ly * lx);
+            double *at = tab.data();
+            auto fill = [&](int m, int ld, bool transposed) {
                 for (int i = 0; i < m; ++i)
                     for (int k = 0; k < m; ++k)
-                        Cm[(size_t)i * m + k] = std::sqrt((k == 0 ? 1.0 : 2.0) / m) * std::cos(pi * k * (2 * i + 1) / (2.0 * m));
+                        at[transposed ? (size_t)k * ld + i : (size_t)i * ld + k] =
+                            std::sqrt((k == 0 ? 1.0 : 2.0) / m) * std::cos(pi * k * (2 * i + 1) / (2.0 * m));
+                at += (size_t)ld * ld;
             };
-            fill(tab.data(), bx);
-            fill(tab.data() + (size_t)bx * bx, by);
-            double *Dinv = tab.data() + (size_t)bx * bx + (size_t)by * by;
+            fill(bx, lx, false);
+            if (c.big_strip) fill(bx, lx, true);
+            fill(by, ly, false);
+            if (c.big_strip) fill(by, ly, true);
+            double *Dinv = at;
             for (int mm = 0; mm < by; ++mm)
                 for (int k = 0; k < bx; ++k) {
                     const double lam = -B.ax * (2.0 - 2.0 * std::cos(pi * k / bx)) - B.ay * (2.0 - 2.0 * std::cos(pi * mm / by));
-                    Dinv[(size_t)mm * bx + k] = (k == 0 && mm == 0) ? 0.0 : 1.0 / lam;
+                    Dinv[(size_t)mm * lx + k] = (k == 0 && mm == 0) ? 0.0 : 1.0 / lam;
                 }
             std::vector<float> tab32(tab.begin(), tab.end());
             ALLOC(&c.big_tab, tab.size()); ALLOC(&c.big_tab32, tab.size());
-            ALLOC(&c.big_work, (size_t)2 * bx * by); ALLOC(&c.big_work32, (size_t)2 * bx * by);
+            ALLOC(&c.big_work, (size_t)2 * lx * ly); ALLOC(&c.big_work32, (size_t)2 * lx * ly);
             hipError_t e1 = hipMemcpy(c.big_tab, tab.data(), tab.size() * 8, hipMemcpyHostToDevice);
             hipError_t e2 = hipMemcpy(c.big_tab32, tab32.data(), tab32.size() * 4, hipMemcpyHostToDevice);
             if (e1 != hipSuccess || e2 != hipSuccess) return bail(AMRESSIF_ERR_HIP, "bottom DCT table upload failed");

@@ -199,6 +199,7 @@ struct Ctx {
     // work arrays (null: the bottom is the dense pseudo-inverse / k_tail_dct)
     double *big_tab = nullptr, *big_work = nullptr;
     float *big_tab32 = nullptr, *big_work32 = nullptr;
+    bool big_strip = false;  // laid out for k_dense_strip
     // FP32 V-cycle: the level above it smoothed inside the same kernel
     // (k_tail_dct_ext; 32, 64 or 128 rows, at most 128 columns)
     int tail_ext = 1;
@@ -301,6 +302,7 @@ hipError_t launch_mg_start(const Ctx &c, int require_mom = 0, const double *us =
 hipError_t launch_poisson_start(const Ctx &c, int mode, int center, const double *phi1, const double *phi2,
                                 double *phi0, int mixed, const double *us = nullptr, const double *vs = nullptr);
 hipError_t launch_fin_resid(const Ctx &c, int nblocks);
+bool bottom_strips(int nx, int ny);  // a dense bottom level solved strip-wise
 hipError_t launch_vcycle(const Ctx &c, int mixed);
 hipError_t launch_vcycle_step(const Ctx &c, int mixed, int par, const double *phi_in, double *phi_out, int *nblocks);
 hipError_t launch_correct_residual(const Ctx &c, const double *phi_in, double *phi_out, int with_correction,

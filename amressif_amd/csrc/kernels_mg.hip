@@ -1782,6 +1782,141 @@ __global__ __launch_bounds__(256) void k_dense_mm(const T *A, int lda, int ta, c
     if (row < M && col < N) C[(size_t)row * ldc + col] = S ? acc * S[(size_t)row * lds + col] : acc;
 }
 
+// The same on the matrix cores, in two launches: C_y (D+ .* (C_y^T (r C_x))) needs only
+// a 16-column strip's own columns up to its last factor, so one launch does three
+// products (a strip per workgroup in LDS, a 16-row tile per wave) and a second one
+// multiplies by C_x^T (a tile per wave).  Latency bound: a tile's whole depth, 128, is
+// loaded at once.  At 125^2 in FP32 10.2 + 4.1 us against 4 x 7.1, in FP64 15.6 + 4.9.
+// Past 128 a strip's products take several rounds of loads on few workgroups: 129^2
+// would take 29 + 4.8 us (FP32) against about 29, 255^2 49 + 7.2 (FP64) against 59.
+constexpr int kStripLd = 20;   // row stride of a strip: four groups of 16 lanes in different banks
+constexpr int kStripWaves = 8;
+constexpr int kStripMax = 128;
+template <class T>
+using dct_v4 = T __attribute__((ext_vector_type(4)));
+template <class T>
+struct Mfma;
+template <>
+struct Mfma<float> {
+    using V = dct_v4f;
+    static __device__ __forceinline__ V mul(float a, float b, V d) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, d, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int lk, int v) { return 4 * lk + v; }
+};
+template <>
+struct Mfma<double> {
+    using V = dct_v4d;
+    static __device__ __forceinline__ V mul(double a, double b, V d) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, d, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int lk, int v) { return lk + 4 * v; }
+};
+
+// One 16 x 16 tile of A B over whole blocks of 128 of k: fa(k, a) reads this lane's
+// A[row][k .. k + 3], fb(k) its B[k][col].  (A block's four instructions take k = 16 kb
+// + 4 (l / 16) + q, so that a lane has four neighbours.)
+template <class T, class FA, class FB>
+__device__ __forceinline__ typename Mfma<T>::V strip_tile(int K, int lk, FA fa, FB fb)
+{
+    typename Mfma<T>::V acc = {0, 0, 0, 0};
+    for (int kb = 0; kb < K; kb += 128) {
+        T a[8][4], b[8][4];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = kb + 16 * u + 4 * lk;
+            fa(k, a[u]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[u][q] = fb(k + q);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc = Mfma<T>::mul(a[u][q], b[u][q], acc);
+    }
+    return acc;
+}
+
+// Tables C_x, C_x^T, C_y, C_y^T, D+ of pitch and rows padded to multiples of 128 with
+// zeros, and W^T of the same shape.  Masked are r, whose row may end in anything, and W^T,
+// whose rows past the last strip are not written.
+// Each is read 16 neighbours to a row (reading C_y and C_x by columns from one copy
+// made the vector caches' line rate the bound, 17 us at 125^2).
+template <class T>
+__global__ __launch_bounds__(64 * kStripWaves) void k_dense_strip(const T *r, int pr, const T *Cx, const T *Cy,
+                                                                  const T *CyT, const T *Dinv, T *WT, int nx, int ny,
+                                                                  int ldx, int ldy, const Ctl *ctl)
+{
+    extern __shared__ __align__(16) unsigned char strip_sh[];
+    if (ctl->mg_done | ctl->gm_stop) return;
+    T *s1 = (T *)strip_sh, *s2 = s1 + ldy * kStripLd;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, li = l & 15, lk = l >> 4;
+    const int col = 16 * blockIdx.x + li;
+    for (int r0 = 16 * w; r0 < ldy; r0 += 16 * kStripWaves) {  // r C_x
+        const T *ra = r + (size_t)pr * min(r0 + li, ny - 1);
+        const auto d = strip_tile<T>(ldx, lk,
+                                     [&](int k, T (&a)[4]) {
+                                         const dct_v4<T> x = *(const dct_v4<T> *)(ra + min(k, pr - 4));
+#pragma unroll
+                                         for (int q = 0; q < 4; ++q) a[q] = k + q < nx ? x[q] : T(0);
+                                     },
+                                     [&](int k) { return Cx[k * ldx + col]; });
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int row = r0 + Mfma<T>::row(lk, v);
+            s1[row * kStripLd + li] = row < ny ? d[v] : T(0);
+        }
+    }
+    __syncthreads();
+    for (int r0 = 16 * w; r0 < ldy; r0 += 16 * kStripWaves) {  // D+ .* (C_y^T .)
+        T dv[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dv[v] = Dinv[(r0 + Mfma<T>::row(lk, v)) * ldx + col];
+        const auto d = strip_tile<T>(ldy, lk,
+                                     [&](int k, T (&a)[4]) {
+#pragma unroll
+                                         for (int q = 0; q < 4; ++q) a[q] = Cy[(k + q) * ldy + r0 + li];
+                                     },
+                                     [&](int k) { return s1[k * kStripLd + li]; });
+#pragma unroll
+        for (int v = 0; v < 4; ++v) s2[(r0 + Mfma<T>::row(lk, v)) * kStripLd + li] = d[v] * dv[v];
+    }
+    __syncthreads();
+    for (int r0 = 16 * w; r0 < ldy; r0 += 16 * kStripWaves) {  // C_y .
+        const auto d = strip_tile<T>(ldy, lk,
+                                     [&](int k, T (&a)[4]) {
+#pragma unroll
+                                         for (int q = 0; q < 4; ++q) a[q] = CyT[(k + q) * ldy + r0 + li];
+                                     },
+                                     [&](int k) { return s2[k * kStripLd + li]; });
+#pragma unroll
+        for (int v = 0; v < 4; ++v) WT[col * ldy + r0 + Mfma<T>::row(lk, v)] = d[v];
+    }
+}
+
+// e = W C_x^T
+template <class T>
+__global__ __launch_bounds__(64) void k_dense_last(const T *WT, const T *CxT, T *e, int pe, int nx, int ny, int ldx,
+                                                   int ldy, const Ctl *ctl)
+{
+    if (ctl->mg_done | ctl->gm_stop) return;
+    const int li = threadIdx.x & 15, lk = threadIdx.x >> 4, r0 = 16 * blockIdx.y;
+    const int col = 16 * blockIdx.x + li;
+    const auto d = strip_tile<T>(ldx, lk,
+                                 [&](int k, T (&a)[4]) {
+#pragma unroll
+                                     for (int q = 0; q < 4; ++q) {
+                                         const T x = WT[(k + q) * ldy + r0 + li];
+                                         a[q] = k + q < nx ? x : T(0);
+                                     }
+                                 },
+                                 [&](int k) { return CxT[k * ldx + col]; });
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int row = r0 + Mfma<T>::row(lk, v);
+        if (row < ny && col < nx) e[(size_t)pe * row + col] = d[v];
+    }
+}
+
+static int round_up128(int n) { return (n + 127) / 128 * 128; }
+bool bottom_strips(int nx, int ny) { return nx <= kStripMax && ny <= kStripMax; }
+
 template <class T>
 static hipError_t dense_bottom(const Ctx &c, const T *r, int pr, T *e, int pe, const Level &L)
 {
@@ -1792,6 +1927,15 @@ static hipError_t dense_bottom(const Ctx &c, const T *r, int pr, T *e, int pe, c
     T *W2 = W1 + (size_t)nx * ny;
     const dim3 grid((nx + 15) / 16, (ny + 15) / 16);
     const Ctl *ctl = c.ctl;
+    if (c.big_strip) {
+        const int lx = round_up128(nx), ly = round_up128(ny);
+        const T *CxT = Cx + (size_t)lx * lx, *Cyp = CxT + (size_t)lx * lx, *CyT = Cyp + (size_t)ly * ly,
+                *D = CyT + (size_t)ly * ly;
+        hipLaunchKernelGGL(k_dense_strip<T>, dim3(grid.x), dim3(64 * kStripWaves), 2 * sizeof(T) * kStripLd * ly, c.stream,
+                           r, pr, Cx, Cyp, CyT, D, W1, nx, ny, lx, ly, ctl);
+        hipLaunchKernelGGL(k_dense_last<T>, grid, dim3(64), 0, c.stream, (const T *)W1, CxT, e, pe, nx, ny, lx, ly, ctl);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_dense_mm<T>, grid, dim3(256), 0, c.stream, r, pr, 0, Cx, nx, 0, W1, nx, ny, nx, nx,
                        (const T *)nullptr, 0, ctl);                                 // r C_x
     hipLaunchKernelGGL(k_dense_mm<T>, grid, dim3(256), 0, c.stream, Cy, ny, 1, (const T *)W1, nx, 0, W2, nx, ny, nx,

@@ -502,6 +502,25 @@ def test_odd_bottom_poisson_solve_matches_the_exact_solve(n):
         assert rel(sol.cpu().numpy()[1:-1, 1:-1], xe[1:-1, 1:-1]) < bar, prec
 
 
+@pytest.mark.parametrize("n", [66, 70, 162, 226, 254, 258])
+def test_odd_bottom_strips_match_the_exact_solve(n):
+    """Odd bottoms of 33, 35, 81, 113, 127 and 129 cells a side: one past two
+    whole 16-column strips, the row tiles' remainders, the last size solved strip
+    by strip and the first one solved by four dense products, in both types."""
+    api = _api()
+    rng = np.random.default_rng(n)
+    rhs = np.zeros((n + 2, n + 2))
+    rhs[1:-1, 1:-1] = rng.standard_normal((n, n))
+    xe, _, _ = Oracle(n, 100.0, 1e-4, poisson="dct").poisson_solve(rhs)
+    for prec, tol, bar in ((0, 1e-12, 1e-9), (1, 1e-10, 1e-7)):
+        ctx = api.Context(api.cavity_inputs(n, 100.0, precision=prec))
+        sol, it, res = ctx.poisson_advance(cuda(rhs), tol_rel=tol)
+        print(f"n={n} prec={prec}: {it} cycles, {res:.1e}")
+        # (two grids with an exact bottom: a bottom that is off costs cycles)
+        assert res <= tol and it <= 16, (prec, it, res)
+        assert rel(sol.cpu().numpy()[1:-1, 1:-1], xe[1:-1, 1:-1]) < bar, prec
+
+
 def test_odd_bottom_steps_match_oracle():
     ref, rs, got, st = run_both(130, 400.0, 4, init="seeded")
     check_step_parity(ref, rs, got, st)
