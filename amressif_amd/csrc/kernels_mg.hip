@@ -1786,10 +1786,11 @@ __global__ __launch_bounds__(256) void k_dense_mm(const T *A, int lda, int ta, c
 // a 16-column strip's own columns up to its last factor, so one launch does three
 // products (a strip per workgroup in LDS, a 16-row tile per wave) and a second one
 // multiplies by C_x^T (a tile per wave).  Latency bound: a tile's whole depth, 128, is
-// loaded at once.  At 125^2 in FP32 10.2 + 4.1 us against 4 x 7.1, in FP64 15.6 + 4.9.
-// Past 128 a strip's products take several rounds of loads on few workgroups: 129^2
-// would take 29 + 4.8 us (FP32) against about 29, 255^2 49 + 7.2 (FP64) against 59.
-constexpr int kStripLd = 20;   // row stride of a strip: four groups of 16 lanes in different banks
+// loaded at once.  At 125^2 in FP32 12.0 + 4.1 us against 4 x 7.1, in FP64 18.6 + 6.5.
+// Past 128 a strip's products take several rounds of loads on few workgroups: with a
+// limit of 256 they took 34 us (FP32) and 52 (FP64) at 191^2 and would at 129^2, where four
+// dense products take about 29.
+constexpr int kStripLd = 16;   // row stride of a strip: four rows of 16 lanes in different banks
 constexpr int kStripWaves = 8;
 constexpr int kStripMax = 128;
 template <class T>
@@ -1809,26 +1810,36 @@ struct Mfma<double> {
     static __device__ __forceinline__ int row(int lk, int v) { return lk + 4 * v; }
 };
 
-// One 16 x 16 tile of A B over whole blocks of 128 of k: fa(k, a) reads this lane's
-// A[row][k .. k + 3], fb(k) its B[k][col].  (A block's four instructions take k = 16 kb
-// + 4 (l / 16) + q, so that a lane has four neighbours.)
+// Four neighbours of a row in each of the four lanes of a column (k = 4 g + q) to one of
+// each quarter in every lane (k = 4 q + g).
+template <class T>
+__device__ __forceinline__ void quad_transpose(T (&x)[4], int g)
+{
+    auto pick = [](const T (&y)[4], int q) {
+        const T lo = q & 1 ? y[1] : y[0], hi = q & 1 ? y[3] : y[2];
+        return q & 2 ? hi : lo;
+    };
+    T v[4];
+    v[0] = pick(x, g);
+#pragma unroll
+    for (int r = 1; r < 4; ++r) v[r] = __shfl_xor(pick(x, g ^ r), 16 * r, 64);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = pick(v, q ^ g);
+}
+
+// One 16 x 16 tile of A B over whole blocks of 128 of k: fa(kb, a) reads this lane's
+// A[row][kb + 4 u + lk], u < 32, fb(k) its B[k][col].  k goes up in order, as in k_dense_mm.
 template <class T, class FA, class FB>
 __device__ __forceinline__ typename Mfma<T>::V strip_tile(int K, int lk, FA fa, FB fb)
 {
     typename Mfma<T>::V acc = {0, 0, 0, 0};
     for (int kb = 0; kb < K; kb += 128) {
-        T a[8][4], b[8][4];
+        T a[32], b[32];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int k = kb + 16 * u + 4 * lk;
-            fa(k, a[u]);
+        for (int u = 0; u < 32; ++u) b[u] = fb(kb + 4 * u + lk);
+        fa(kb, a);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) b[u][q] = fb(k + q);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc = Mfma<T>::mul(a[u][q], b[u][q], acc);
+        for (int u = 0; u < 32; ++u) acc = Mfma<T>::mul(a[u], b[u], acc);
     }
     return acc;
 }
@@ -1851,10 +1862,21 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_dense_strip(const T *r, in
     for (int r0 = 16 * w; r0 < ldy; r0 += 16 * kStripWaves) {  // r C_x
         const T *ra = r + (size_t)pr * min(r0 + li, ny - 1);
         const auto d = strip_tile<T>(ldx, lk,
-                                     [&](int k, T (&a)[4]) {
-                                         const dct_v4<T> x = *(const dct_v4<T> *)(ra + min(k, pr - 4));
+                                     [&](int kb, T (&a)[32]) {
+                                         dct_v4<T> x[8];
 #pragma unroll
-                                         for (int q = 0; q < 4; ++q) a[q] = k + q < nx ? x[q] : T(0);
+                                         for (int u = 0; u < 8; ++u)
+                                             x[u] = *(const dct_v4<T> *)(ra + min(kb + 16 * u + 4 * lk, pr - 4));
+#pragma unroll
+                                         for (int u = 0; u < 8; ++u) {
+                                             T y[4];
+#pragma unroll
+                                             for (int q = 0; q < 4; ++q)
+                                                 y[q] = kb + 16 * u + 4 * lk + q < nx ? x[u][q] : T(0);
+                                             quad_transpose(y, lk);
+#pragma unroll
+                                             for (int q = 0; q < 4; ++q) a[4 * u + q] = y[q];
+                                         }
                                      },
                                      [&](int k) { return Cx[k * ldx + col]; });
 #pragma unroll
@@ -1869,9 +1891,9 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_dense_strip(const T *r, in
 #pragma unroll
         for (int v = 0; v < 4; ++v) dv[v] = Dinv[(r0 + Mfma<T>::row(lk, v)) * ldx + col];
         const auto d = strip_tile<T>(ldy, lk,
-                                     [&](int k, T (&a)[4]) {
+                                     [&](int kb, T (&a)[32]) {
 #pragma unroll
-                                         for (int q = 0; q < 4; ++q) a[q] = Cy[(k + q) * ldy + r0 + li];
+                                         for (int u = 0; u < 32; ++u) a[u] = Cy[(kb + 4 * u + lk) * ldy + r0 + li];
                                      },
                                      [&](int k) { return s1[k * kStripLd + li]; });
 #pragma unroll
@@ -1880,9 +1902,9 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_dense_strip(const T *r, in
     __syncthreads();
     for (int r0 = 16 * w; r0 < ldy; r0 += 16 * kStripWaves) {  // C_y .
         const auto d = strip_tile<T>(ldy, lk,
-                                     [&](int k, T (&a)[4]) {
+                                     [&](int kb, T (&a)[32]) {
 #pragma unroll
-                                         for (int q = 0; q < 4; ++q) a[q] = CyT[(k + q) * ldy + r0 + li];
+                                         for (int u = 0; u < 32; ++u) a[u] = CyT[(kb + 4 * u + lk) * ldy + r0 + li];
                                      },
                                      [&](int k) { return s2[k * kStripLd + li]; });
 #pragma unroll
@@ -1899,11 +1921,12 @@ __global__ __launch_bounds__(64) void k_dense_last(const T *WT, const T *CxT, T 
     const int li = threadIdx.x & 15, lk = threadIdx.x >> 4, r0 = 16 * blockIdx.y;
     const int col = 16 * blockIdx.x + li;
     const auto d = strip_tile<T>(ldx, lk,
-                                 [&](int k, T (&a)[4]) {
+                                 [&](int kb, T (&a)[32]) {
 #pragma unroll
-                                     for (int q = 0; q < 4; ++q) {
-                                         const T x = WT[(k + q) * ldy + r0 + li];
-                                         a[q] = k + q < nx ? x : T(0);
+                                     for (int u = 0; u < 32; ++u) {
+                                         const int k = kb + 4 * u + lk;
+                                         const T x = WT[k * ldy + r0 + li];
+                                         a[u] = k < nx ? x : T(0);
                                      }
                                  },
                                  [&](int k) { return CxT[k * ldx + col]; });
