@@ -1117,20 +1117,22 @@ int amressif_load_state(amressif_ctx *ctx, const amr_array4 velCont[2], const am
     if (ctx && ctx->c.gen) return amr_gen_load_state(ctx, velCont, velContPrev, userCtx);
     if (!ctx || !velCont || !velContPrev) return fail(ctx, AMRESSIF_ERR_ARG, "null argument");
     Ctx &c = ctx->c;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &velCont[d], d, "velCont")) return rc;
         if (int rc = check_face(ctx, &velContPrev[d], d, "velContPrev")) return rc;
-        HIPCHK(amr::launch_pack_face(c, velCont[d], c.U[d], d));
-        HIPCHK(amr::launch_pack_face(c, velContPrev[d], c.Uprev[d], d));
+        pk.face(c, velCont[d], c.U[d], d);
+        pk.face(c, velContPrev[d], c.Uprev[d], d);
     }
     if (userCtx) {
         if (int rc = check_cell(ctx, userCtx, 2, "userCtx")) return rc;
-        HIPCHK(amr::launch_pack_cell(c, *userCtx, 0, c.p));
-        HIPCHK(amr::launch_pack_cell(c, *userCtx, 1, c.phi));
+        pk.cell(c, *userCtx, 0, c.p);
+        pk.cell(c, *userCtx, 1, c.phi);
     } else {
         HIPCHK(amr::launch_fill(c, c.p, (int64_t)(c.g.n + 1) * c.g.P, 0.0));
         HIPCHK(amr::launch_fill(c, c.phi, (int64_t)(c.g.n + 1) * c.g.P, 0.0));
     }
+    HIPCHK(amr::launch_pack(c, pk));
     HIPCHK(amr::launch_mg_start(c));  // phi_mean = 0 for the loaded phi
     c.phih_valid = 0;                  // no solution history for the warm start
     c.pred_valid = 0;
@@ -1146,16 +1148,18 @@ int amressif_store_state(const amressif_ctx *cctx, amr_array4 velCont[2], amr_ar
     amressif_ctx *ctx = const_cast<amressif_ctx *>(cctx);
     if (!ctx) return AMRESSIF_ERR_ARG;
     Ctx &c = ctx->c;
+    amr::Copies out;
     for (int d = 0; d < 2; ++d) {
         if (velCont) {
             if (int rc = check_face(ctx, &velCont[d], d, "velCont")) return rc;
-            HIPCHK(amr::launch_unpack_face(c, c.U[d], velCont[d], d));
+            out.face(c, velCont[d], c.U[d], d);
         }
         if (velContPrev) {
             if (int rc = check_face(ctx, &velContPrev[d], d, "velContPrev")) return rc;
-            HIPCHK(amr::launch_unpack_face(c, c.Uprev[d], velContPrev[d], d));
+            out.face(c, velContPrev[d], c.Uprev[d], d);
         }
     }
+    HIPCHK(amr::launch_unpack(c, out));
     if (userCtx) {
         if (int rc = check_cell(ctx, userCtx, 2, "userCtx")) return rc;
         HIPCHK(amr::launch_unpack_cell_shift(c, c.p, *userCtx, 0, 1, nullptr));
@@ -1558,11 +1562,13 @@ int amressif_cont2cart(amressif_ctx *ctx, const amr_array4 velCont[2], amr_array
     if (!ctx || !velCont) return fail(ctx, AMRESSIF_ERR_ARG, "null argument");
     Ctx &c = ctx->c;
     if (int rc = ensure_module_scratch(ctx)) return rc;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &velCont[d], d, "velCont")) return rc;
-        HIPCHK(amr::launch_pack_face(c, velCont[d], c.M[0][d], d));
+        pk.face(c, velCont[d], c.M[0][d], d);
     }
     if (int rc = check_cell(ctx, velCart, 2, "velCart")) return rc;
+    HIPCHK(amr::launch_pack(c, pk));
     HIPCHK(amr::launch_cont2cart_out(c, c.M[0][0], c.M[0][1], *velCart));
     HIPCHK(hipStreamSynchronize(c.stream));
     return AMRESSIF_OK;
@@ -1576,20 +1582,24 @@ int amressif_momentum_rhs(amressif_ctx *ctx, const amr_array4 velStar[2], const 
     if (!ctx || !velStar || !userCtx || !rhs) return fail(ctx, AMRESSIF_ERR_ARG, "null argument");
     Ctx &c = ctx->c;
     if (int rc = ensure_module_scratch(ctx)) return rc;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &velStar[d], d, "velStar")) return rc;
         if (int rc = check_face(ctx, &rhs[d], d, "rhs")) return rc;
-        HIPCHK(amr::launch_pack_face(c, velStar[d], c.M[0][d], d));
+        pk.face(c, velStar[d], c.M[0][d], d);
     }
     if (int rc = check_cell(ctx, userCtx, 1, "userCtx")) return rc;
-    HIPCHK(amr::launch_pack_cell(c, *userCtx, 0, c.Mc[0]));
+    pk.cell(c, *userCtx, 0, c.Mc[0]);
+    HIPCHK(amr::launch_pack(c, pk));
     amr::StageLaunch a{};
     a.us = c.M[0][0]; a.vs = c.M[0][1]; a.p = c.Mc[0];
     a.uo = c.M[1][0]; a.vo = c.M[1][1];
     a.mode = 2;
     int nb = 0;
     HIPCHK(amr::launch_stage(c, a, &nb));
-    for (int d = 0; d < 2; ++d) HIPCHK(amr::launch_unpack_face(c, c.M[1][d], rhs[d], d));
+    amr::Copies out;
+    for (int d = 0; d < 2; ++d) out.face(c, rhs[d], c.M[1][d], d);
+    HIPCHK(amr::launch_unpack(c, out));
     HIPCHK(hipStreamSynchronize(c.stream));
     return AMRESSIF_OK;
 }
@@ -1604,19 +1614,22 @@ int amressif_rk_stage(amressif_ctx *ctx, int sub, amr_array4 velStar[2], const a
     if (sub < 0 || sub > 3) return fail(ctx, AMRESSIF_ERR_ARG, "sub must be 0..3");
     Ctx &c = ctx->c;
     if (int rc = ensure_module_scratch(ctx)) return rc;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &velStar[d], d, "velStar")) return rc;
         if (int rc = check_face(ctx, &velCont[d], d, "velCont")) return rc;
         if (int rc = check_face(ctx, &velContPrev[d], d, "velContPrev")) return rc;
         if (int rc = check_face(ctx, &velContPrevPrev[d], d, "velContPrevPrev")) return rc;
-        HIPCHK(amr::launch_pack_face(c, velStar[d], c.M[0][d], d));
-        HIPCHK(amr::launch_pack_face(c, velCont[d], c.M[1][d], d));
-        HIPCHK(amr::launch_pack_face(c, velContPrev[d], c.M[2][d], d));
-        HIPCHK(amr::launch_pack_face(c, velContPrevPrev[d], c.M[3][d], d));
-        HIPCHK(amr::launch_bdf2_const(c, c.M[2][d], c.M[3][d], c.M[2][d], d));  // in place: c from (u^n, u^{n-1})
+        pk.face(c, velStar[d], c.M[0][d], d);
+        pk.face(c, velCont[d], c.M[1][d], d);
+        pk.face(c, velContPrev[d], c.M[2][d], d);
+        pk.face(c, velContPrevPrev[d], c.M[3][d], d);
     }
     if (int rc = check_cell(ctx, userCtx, 1, "userCtx")) return rc;
-    HIPCHK(amr::launch_pack_cell(c, *userCtx, 0, c.Mc[0]));
+    pk.cell(c, *userCtx, 0, c.Mc[0]);
+    HIPCHK(amr::launch_pack(c, pk));
+    for (int d = 0; d < 2; ++d)  // in place: c from (u^n, u^{n-1})
+        HIPCHK(amr::launch_bdf2_const(c, c.M[2][d], c.M[3][d], c.M[2][d], d));
     amr::StageLaunch a{};
     a.us = c.M[0][0]; a.vs = c.M[0][1];
     a.ub = c.M[1][0]; a.vb = c.M[1][1];
@@ -1628,7 +1641,9 @@ int amressif_rk_stage(amressif_ctx *ctx, int sub, amr_array4 velStar[2], const a
     HIPCHK(amr::launch_ctl_reset_step(c));  // clears mom_done so the guarded kernel runs
     int nb = 0;
     HIPCHK(amr::launch_stage(c, a, &nb));
-    for (int d = 0; d < 2; ++d) HIPCHK(amr::launch_unpack_face(c, c.M[3][d], velStar[d], d));
+    amr::Copies out;
+    for (int d = 0; d < 2; ++d) out.face(c, velStar[d], c.M[3][d], d);
+    HIPCHK(amr::launch_unpack(c, out));
     HIPCHK(hipStreamSynchronize(c.stream));
     return AMRESSIF_OK;
 }
@@ -1643,33 +1658,36 @@ int amressif_fluxes(amressif_ctx *ctx, const amr_array4 velStar[2], amr_array4 *
         return fail(ctx, AMRESSIF_ERR_ARG, "fluxHalfN1 and fluxHalfN2 go together");
     Ctx &c = ctx->c;
     if (int rc = ensure_module_scratch(ctx)) return rc;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &velStar[d], d, "velStar")) return rc;
         if (fluxHalfN1) {
             if (int rc = check_face(ctx, &fluxHalfN1[d], d, "fluxHalfN1")) return rc;
             if (int rc = check_face(ctx, &fluxHalfN2[d], d, "fluxHalfN2")) return rc;
         }
-        HIPCHK(amr::launch_pack_face(c, velStar[d], c.M[0][d], d));
+        pk.face(c, velStar[d], c.M[0][d], d);
     }
     if (fluxConvect)
         if (int rc = check_cell(ctx, fluxConvect, 2, "fluxConvect")) return rc;
     if (fluxViscous)
         if (int rc = check_cell(ctx, fluxViscous, 2, "fluxViscous")) return rc;
     // M[1]: fluxHalfN1 (x-, y-faces), M[2]: fluxHalfN2, Mc: fluxConvect, M[3]: fluxViscous
+    HIPCHK(amr::launch_pack(c, pk));
     const bool half = fluxHalfN1 != nullptr;
     HIPCHK(amr::launch_flux_fields(c, c.M[0][0], c.M[0][1], half ? c.M[1][0] : nullptr, half ? c.M[2][0] : nullptr,
                                    half ? c.M[1][1] : nullptr, half ? c.M[2][1] : nullptr,
                                    fluxConvect ? c.Mc[0] : nullptr, fluxConvect ? c.Mc[1] : nullptr,
                                    fluxViscous ? c.M[3][0] : nullptr, fluxViscous ? c.M[3][1] : nullptr));
-    if (half)
-        for (int d = 0; d < 2; ++d) {
-            HIPCHK(amr::launch_unpack_face(c, c.M[1][d], fluxHalfN1[d], d));
-            HIPCHK(amr::launch_unpack_face(c, c.M[2][d], fluxHalfN2[d], d));
+    amr::Copies out;
+    for (int d = 0; d < 2; ++d) {
+        if (half) {
+            out.face(c, fluxHalfN1[d], c.M[1][d], d);
+            out.face(c, fluxHalfN2[d], c.M[2][d], d);
         }
-    for (int comp = 0; comp < 2; ++comp) {
-        if (fluxConvect) HIPCHK(amr::launch_unpack_cell(c, c.Mc[comp], *fluxConvect, comp, 0));
-        if (fluxViscous) HIPCHK(amr::launch_unpack_cell(c, c.M[3][comp], *fluxViscous, comp, 0));
+        if (fluxConvect) out.cell(c, *fluxConvect, d, c.Mc[d]);
+        if (fluxViscous) out.cell(c, *fluxViscous, d, c.M[3][d]);
     }
+    HIPCHK(amr::launch_unpack(c, out));
     HIPCHK(hipStreamSynchronize(c.stream));
     return AMRESSIF_OK;
 }
@@ -1681,12 +1699,14 @@ int amressif_pseudo_norm(amressif_ctx *ctx, const amr_array4 velCont[2], const a
     if (!ctx || !velCont || !velStar || !norm) return fail(ctx, AMRESSIF_ERR_ARG, "null argument");
     Ctx &c = ctx->c;
     if (int rc = ensure_module_scratch(ctx)) return rc;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &velCont[d], d, "velCont")) return rc;
         if (int rc = check_face(ctx, &velStar[d], d, "velStar")) return rc;
-        HIPCHK(amr::launch_pack_face(c, velCont[d], c.M[0][d], d));
-        HIPCHK(amr::launch_pack_face(c, velStar[d], c.M[1][d], d));
+        pk.face(c, velCont[d], c.M[0][d], d);
+        pk.face(c, velStar[d], c.M[1][d], d);
     }
+    HIPCHK(amr::launch_pack(c, pk));
     HIPCHK(amr::launch_norm(c, c.M[0][0], c.M[0][1], c.M[1][0], c.M[1][1], c.dscalar));
     HIPCHK(hipMemcpyAsync(norm, c.dscalar, 8, hipMemcpyDeviceToHost, c.stream));
     HIPCHK(hipStreamSynchronize(c.stream));
@@ -1701,11 +1721,13 @@ int amressif_poisson_rhs(amressif_ctx *ctx, const amr_array4 vel[2], amr_array4 
     if (!ctx || !vel || !rhs) return fail(ctx, AMRESSIF_ERR_ARG, "null argument");
     Ctx &c = ctx->c;
     if (int rc = ensure_module_scratch(ctx)) return rc;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &vel[d], d, "vel")) return rc;
-        HIPCHK(amr::launch_pack_face(c, vel[d], c.M[0][d], d));
+        pk.face(c, vel[d], c.M[0][d], d);
     }
     if (int rc = check_cell(ctx, rhs, 1, "rhs")) return rc;
+    HIPCHK(amr::launch_pack(c, pk));
     int nb = 0;
     HIPCHK(amr::launch_poisson_rhs(c, c.M[0][0], c.M[0][1], c.Mc[0], &nb));
     HIPCHK(amr::launch_fin_prhs(c, nb));
@@ -1727,7 +1749,9 @@ int amressif_poisson_solve(amressif_ctx *ctx, amr_array4 *sol, const amr_array4 
     if (int rc = check_cell(ctx, sol, 1, "sol")) return rc;
     if (int rc = ensure_module_scratch(ctx)) return rc;
     HIPCHK(amr::launch_ctl_set(c, c.in.momentum_tolerance, tol_rel, tol_abs, c.in.IterNum, c.in.mg_max_iter));
-    HIPCHK(amr::launch_pack_cell(c, *rhs, 0, c.b));
+    amr::Copies pk;
+    pk.cell(c, *rhs, 0, c.b);
+    HIPCHK(amr::launch_pack(c, pk));
     HIPCHK(amr::launch_mean_b(c, c.b));
     HIPCHK(amr::launch_center_b(c, c.b));
     if (int rc = poisson_loop(ctx)) return rc;
@@ -1750,18 +1774,22 @@ int amressif_project(amressif_ctx *ctx, const amr_array4 velStar[2], amr_array4 
     if (!ctx || !velStar || !userCtx || !velCont) return fail(ctx, AMRESSIF_ERR_ARG, "null argument");
     Ctx &c = ctx->c;
     if (int rc = ensure_module_scratch(ctx)) return rc;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (int rc = check_face(ctx, &velStar[d], d, "velStar")) return rc;
         if (int rc = check_face(ctx, &velCont[d], d, "velCont")) return rc;
-        HIPCHK(amr::launch_pack_face(c, velStar[d], c.M[0][d], d));
+        pk.face(c, velStar[d], c.M[0][d], d);
     }
     if (int rc = check_cell(ctx, userCtx, 2, "userCtx")) return rc;
-    HIPCHK(amr::launch_pack_cell(c, *userCtx, 0, c.Mc[0]));
-    HIPCHK(amr::launch_pack_cell(c, *userCtx, 1, c.Mc[1]));
+    pk.cell(c, *userCtx, 0, c.Mc[0]);
+    pk.cell(c, *userCtx, 1, c.Mc[1]);
+    HIPCHK(amr::launch_pack(c, pk));
     int nb = 0;
     HIPCHK(amr::launch_project_ex(c, c.M[0][0], c.M[0][1], c.M[1][0], c.M[1][1], c.Mc[0], c.Mc[1], 0, &nb));
     HIPCHK(amr::launch_fin_project(c, nb, -1));
-    for (int d = 0; d < 2; ++d) HIPCHK(amr::launch_unpack_face(c, c.M[1][d], velCont[d], d));
+    amr::Copies out;
+    for (int d = 0; d < 2; ++d) out.face(c, velCont[d], c.M[1][d], d);
+    HIPCHK(amr::launch_unpack(c, out));
     HIPCHK(amr::launch_unpack_cell(c, c.Mc[0], *userCtx, 0, 1));
     if (int rc = poll(ctx)) return rc;
     if (div_linf) *div_linf = c.ctl_host->div_new;
@@ -2087,26 +2115,28 @@ int amressif_load_dual(amressif_ctx *ctx, const amr_array4 du[2], const amr_arra
     if (int rc = ensure_adjoint(ctx)) return rc;
     Ctx &c = ctx->c;
     const int64_t fsz = (int64_t)(c.g.n + 1) * c.g.P;
+    amr::Copies pk;
     for (int d = 0; d < 2; ++d) {
         if (du) {
             if (int rc = check_face(ctx, &du[d], d, "du")) return rc;
-            HIPCHK(amr::launch_pack_face(c, du[d], c.Du[d], d));
+            pk.face(c, du[d], c.Du[d], d);
         } else {
             HIPCHK(amr::launch_fill(c, c.Du[d], fsz, 0.0));
         }
         if (du_prev) {
             if (int rc = check_face(ctx, &du_prev[d], d, "du_prev")) return rc;
-            HIPCHK(amr::launch_pack_face(c, du_prev[d], c.Dup[d], d));
+            pk.face(c, du_prev[d], c.Dup[d], d);
         } else {
             HIPCHK(amr::launch_fill(c, c.Dup[d], fsz, 0.0));
         }
     }
     if (dp) {
         if (int rc = check_cell(ctx, dp, 1, "dp")) return rc;
-        HIPCHK(amr::launch_pack_cell(c, *dp, 0, c.Dp));
+        pk.cell(c, *dp, 0, c.Dp);
     } else {
         HIPCHK(amr::launch_fill(c, c.Dp, fsz, 0.0));
     }
+    HIPCHK(amr::launch_pack(c, pk));
     if (dlid)
         HIPCHK(hipMemcpyAsync(c.Dlid, dlid, sizeof(double) * c.g.n, hipMemcpyDeviceToDevice, c.stream));
     else
@@ -2122,16 +2152,18 @@ int amressif_store_dual(amressif_ctx *ctx, amr_array4 du[2], amr_array4 du_prev[
     if (!ctx) return AMRESSIF_ERR_ARG;
     Ctx &c = ctx->c;
     if (!c.adj) return fail(ctx, AMRESSIF_ERR_ARG, "no dual state");
+    amr::Copies out;
     for (int d = 0; d < 2; ++d) {
         if (du) {
             if (int rc = check_face(ctx, &du[d], d, "du")) return rc;
-            HIPCHK(amr::launch_unpack_face(c, c.Du[d], du[d], d));
+            out.face(c, du[d], c.Du[d], d);
         }
         if (du_prev) {
             if (int rc = check_face(ctx, &du_prev[d], d, "du_prev")) return rc;
-            HIPCHK(amr::launch_unpack_face(c, c.Dup[d], du_prev[d], d));
+            out.face(c, du_prev[d], c.Dup[d], d);
         }
     }
+    HIPCHK(amr::launch_unpack(c, out));
     if (dp) {
         if (int rc = check_cell(ctx, dp, 1, "dp")) return rc;
         HIPCHK(amr::launch_unpack_cell_shift(c, c.Dp, *dp, 0, 1, nullptr));

@@ -312,9 +312,29 @@ hipError_t configure_tail(Ctx &c);
 hipError_t launch_smooth_fine(const Ctx &c, int kind, double *scratch_phi);
 hipError_t launch_fin_project(const Ctx &c, int nblocks, int step_index, int reset_next = 0, int gated = 0);
 hipError_t launch_cont2cart_out(const Ctx &c, const double *u, const double *v, const amr_array4 &vc);
-hipError_t launch_pack_face(const Ctx &c, const amr_array4 &a, double *dst, int dir);
-hipError_t launch_unpack_face(const Ctx &c, const double *src, const amr_array4 &a, int dir);
-hipError_t launch_pack_cell(const Ctx &c, const amr_array4 &a, int comp, double *dst);
+// Conversions between Array4 views and pitched arrays, one launch for a list (the views must
+// live until it); unpack: shift (device) is subtracted
+constexpr int kCopyMax = 10;
+struct Copies {
+    struct Item {
+        const amr_array4 *a;
+        const double *p, *shift;
+        int comp, nx, ny;
+    };
+    Item it[kCopyMax];
+    int count = 0;
+    void face(const Ctx &c, const amr_array4 &a, const double *p, int dir);
+    void cell(const Ctx &c, const amr_array4 &a, int comp, const double *p, const double *shift = nullptr);
+
+private:
+    void add(const amr_array4 &a, int comp, const double *p, int nx, int ny, const double *shift)
+    {
+        if (count < kCopyMax) it[count] = {&a, p, shift, comp, nx, ny};
+        ++count;  // (one too many: the launch fails)
+    }
+};
+hipError_t launch_pack(const Ctx &c, const Copies &b);
+hipError_t launch_unpack(const Ctx &c, const Copies &b);
 hipError_t launch_unpack_cell(const Ctx &c, const double *src, const amr_array4 &a, int comp, int fill_ghosts);
 // window [i0, i1] x [j0, j1] (global indices, inclusive) of one box view <-> pitched array
 hipError_t launch_pack_window(const Ctx &c, const amr_array4 &a, int comp, double *dst, int i0, int j0, int i1,

@@ -690,20 +690,33 @@ static A4 make_a4(const amr_array4 &a)
     return r;
 }
 
-__global__ __launch_bounds__(256) void k_pack(A4 a, int comp, double *dst, int nx, int ny, int P)
+// The arrays of one call together, one to a grid plane: a module call converts up to
+// nine, and a launch for each is 3 us of which little is the copy (640^2: an RK stage's
+// eleven launches were 4 us apart).
+struct CopyItem {
+    A4 a;
+    double *p;            // pitched
+    const double *shift;  // unpack: subtracted (or null)
+    int comp, nx, ny;
+};
+struct CopyItems {
+    CopyItem it[kCopyMax];
+};
+__global__ __launch_bounds__(256) void k_pack(CopyItems b, int P)
 {
+    const CopyItem &t = b.it[blockIdx.z];
     const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (i >= nx || j >= ny) return;
-    dst[i + (size_t)P * j] = a.ptr[(i - a.lo0) + a.js * (j - a.lo1) + a.ns * comp];
+    if (i >= t.nx || j >= t.ny) return;
+    t.p[i + (size_t)P * j] = t.a.ptr[(i - t.a.lo0) + t.a.js * (j - t.a.lo1) + t.a.ns * t.comp];
 }
 
-__global__ __launch_bounds__(256) void k_unpack(A4 a, int comp, const double *src, int nx, int ny, int P,
-                                                const double *shift)
+__global__ __launch_bounds__(256) void k_unpack(CopyItems b, int P)
 {
+    const CopyItem &t = b.it[blockIdx.z];
     const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (i >= nx || j >= ny) return;
-    const double s = shift ? *shift : 0.0;
-    a.ptr[(i - a.lo0) + a.js * (j - a.lo1) + a.ns * comp] = src[i + (size_t)P * j] - s;
+    if (i >= t.nx || j >= t.ny) return;
+    const double s = t.shift ? *t.shift : 0.0;
+    t.a.ptr[(i - t.a.lo0) + t.a.js * (j - t.a.lo1) + t.a.ns * t.comp] = t.p[i + (size_t)P * j] - s;
 }
 
 // cells including the ghosts the view holds: Neumann mirror in both
@@ -760,29 +773,33 @@ hipError_t launch_unpack_window(const Ctx &c, const double *src, const amr_array
     return hipGetLastError();
 }
 
-hipError_t launch_pack_face(const Ctx &c, const amr_array4 &a, double *dst, int dir)
+void Copies::face(const Ctx &c, const amr_array4 &a, const double *p, int dir)
 {
-    const int n = c.g.n, nx = dir == 0 ? n + 1 : n, ny = dir == 0 ? n : n + 1;
-    hipLaunchKernelGGL(k_pack, dim3((nx + 63) / 64, (ny + 3) / 4), dim3(256), 0, c.stream, make_a4(a), 0, dst, nx,
-                       ny, c.g.P);
-    return hipGetLastError();
+    add(a, 0, p, dir == 0 ? c.g.n + 1 : c.g.n, dir == 0 ? c.g.n : c.g.n + 1, nullptr);
 }
 
-hipError_t launch_unpack_face(const Ctx &c, const double *src, const amr_array4 &a, int dir)
+void Copies::cell(const Ctx &c, const amr_array4 &a, int comp, const double *p, const double *shift)
 {
-    const int n = c.g.n, nx = dir == 0 ? n + 1 : n, ny = dir == 0 ? n : n + 1;
-    hipLaunchKernelGGL(k_unpack, dim3((nx + 63) / 64, (ny + 3) / 4), dim3(256), 0, c.stream, make_a4(a), 0, src,
-                       nx, ny, c.g.P, (const double *)nullptr);
-    return hipGetLastError();
+    add(a, comp, p, c.g.n, c.g.n, shift);
 }
 
-hipError_t launch_pack_cell(const Ctx &c, const amr_array4 &a, int comp, double *dst)
+static hipError_t launch_copies(const Ctx &c, const Copies &b, void (*kern)(CopyItems, int))
 {
-    const int n = c.g.n;
-    hipLaunchKernelGGL(k_pack, dim3((n + 63) / 64, (n + 3) / 4), dim3(256), 0, c.stream, make_a4(a), comp, dst, n,
-                       n, c.g.P);
+    if (b.count == 0) return hipSuccess;
+    if (b.count > kCopyMax) return hipErrorInvalidValue;
+    CopyItems t{};
+    int nx = 0, ny = 0;
+    for (int q = 0; q < b.count; ++q) {
+        const Copies::Item &s = b.it[q];
+        t.it[q] = {make_a4(*s.a), const_cast<double *>(s.p), s.shift, s.comp, s.nx, s.ny};
+        nx = std::max(nx, s.nx);
+        ny = std::max(ny, s.ny);
+    }
+    hipLaunchKernelGGL(kern, dim3((nx + 63) / 64, (ny + 3) / 4, b.count), dim3(256), 0, c.stream, t, c.g.P);
     return hipGetLastError();
 }
+hipError_t launch_pack(const Ctx &c, const Copies &b) { return launch_copies(c, b, k_pack); }
+hipError_t launch_unpack(const Ctx &c, const Copies &b) { return launch_copies(c, b, k_unpack); }
 
 hipError_t launch_unpack_cell_shift(const Ctx &c, const double *src, const amr_array4 &a, int comp,
                                     int fill_ghosts, const double *shift)
@@ -793,8 +810,9 @@ hipError_t launch_unpack_cell_shift(const Ctx &c, const double *src, const amr_a
         hipLaunchKernelGGL(k_unpack_cell_ghosts, dim3((wx + 63) / 64, (wy + 3) / 4), dim3(256), 0, c.stream,
                            make_a4(a), comp, src, n, c.g.P, shift);
     } else {
-        hipLaunchKernelGGL(k_unpack, dim3((n + 63) / 64, (n + 3) / 4), dim3(256), 0, c.stream, make_a4(a), comp,
-                           src, n, n, c.g.P, shift);
+        Copies b;
+        b.cell(c, a, comp, src, shift);
+        return launch_unpack(c, b);
     }
     return hipGetLastError();
 }
