@@ -1851,6 +1851,7 @@ int amressif_time_kernel(amressif_ctx *ctx, int which, int reps, int64_t copy_by
     if ((which == 3 || which == 4 || which == 10) && c.in.precision != AMRESSIF_MIXED)
         return fail(ctx, AMRESSIF_ERR_ARG, "which = 3, 4, 10 need a mixed-precision context");
     if (which == 10 && !amr::mixed_pair_fits(c)) return fail(ctx, AMRESSIF_ERR_ARG, "no one-pass mixed kernel at this size");
+    if (which == 11 && !amr::iteration_fits(c)) return fail(ctx, AMRESSIF_ERR_ARG, "no one-launch pseudo-iteration at this size");
     auto launch = [&]() -> hipError_t {
         if (which == 10) {  // the mixed iteration in one pass, u^k from U into S2
             amr::MixedPairLaunch m{};

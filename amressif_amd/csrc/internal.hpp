@@ -254,7 +254,8 @@ hipError_t launch_stage(const Ctx &c, const StageLaunch &a, int *nblocks);
 hipError_t launch_stage_pair(const Ctx &c, const StageLaunch &a, int *nblocks);
 bool stage_pair_fits(const Ctx &c);
 // one pseudo-iteration in one launch (k_iter_tile) from the base a.ub, a.vb into a.uo, a.vo
-bool iter_tile_wanted(const Ctx &c);
+bool iteration_fits(const Ctx &c);    // its records fit the partials buffer (launch_iteration refuses others)
+bool iter_tile_wanted(const Ctx &c);  // and the step runs it
 hipError_t launch_iteration(const Ctx &c, const StageLaunch &a, int *nblocks);
 const double *iteration_partials(const Ctx &c, int it);  // the norm records of launch `it` of a step
 // cu, cv += -G p on the interior faces, once per FP64 step (p fixed over its pseudo-iterations)

@@ -316,13 +316,16 @@ hipError_t launch_iter_tile(IterTile a, hipStream_t s)
     return hipGetLastError();
 }
 
+// a record of two doubles per workgroup, two sets of them in c.partials (n <= 10239)
+bool iteration_fits(const Ctx &c) { return c.g.n >= 4 && iter_tile_blocks(c.g.n) <= kMaxPartials; }
+
 // The sizes at which a pseudo-iteration runs as one k_iter_tile launch: measured
 // against the two k_stage_pair launches, 18 against 59 us up to 256^2, 30 against 60
 // at 512^2, 48 against 65 at 768^2, 66 against 69 at 1024^2; above, the halo's
 // recomputation costs more than the march (103 against 73 us at 1280^2).
 bool iter_tile_wanted(const Ctx &c)
 {
-    return c.iter_tile && c.g.n >= 4 && (c.g.n <= 1024 || c.iter_tile == 2) && iter_tile_blocks(c.g.n) <= kMaxPartials;
+    return c.iter_tile && iteration_fits(c) && (c.g.n <= 1024 || c.iter_tile == 2);
 }
 
 constexpr int kHalf = 2 * kMaxPartials;  // doubles; c.partials holds twice as many
@@ -331,6 +334,7 @@ const double *iteration_partials(const Ctx &c, int it) { return c.partials + (it
 hipError_t launch_iteration(const Ctx &c, const StageLaunch &s, int *nblocks)
 {
     const Geometry &g = c.g;
+    if (!iteration_fits(c)) return hipErrorInvalidValue;
     IterTile a{};
     a.u = s.ub; a.v = s.vb;
     a.cu = s.cu; a.cv = s.cv;
