@@ -1679,13 +1679,14 @@ int amressif_fluxes(amressif_ctx *ctx, const amr_array4 velStar[2], amr_array4 *
                                    fluxConvect ? c.Mc[0] : nullptr, fluxConvect ? c.Mc[1] : nullptr,
                                    fluxViscous ? c.M[3][0] : nullptr, fluxViscous ? c.M[3][1] : nullptr));
     amr::Copies out;
-    for (int d = 0; d < 2; ++d) {
-        if (half) {
+    if (half)
+        for (int d = 0; d < 2; ++d) {
             out.face(c, fluxHalfN1[d], c.M[1][d], d);
             out.face(c, fluxHalfN2[d], c.M[2][d], d);
         }
-        if (fluxConvect) out.cell(c, *fluxConvect, d, c.Mc[d]);
-        if (fluxViscous) out.cell(c, *fluxViscous, d, c.M[3][d]);
+    for (int comp = 0; comp < 2; ++comp) {
+        if (fluxConvect) out.cell(c, *fluxConvect, comp, c.Mc[comp]);
+        if (fluxViscous) out.cell(c, *fluxViscous, comp, c.M[3][comp]);
     }
     HIPCHK(amr::launch_unpack(c, out));
     HIPCHK(hipStreamSynchronize(c.stream));

@@ -314,7 +314,8 @@ hipError_t launch_smooth_fine(const Ctx &c, int kind, double *scratch_phi);
 hipError_t launch_fin_project(const Ctx &c, int nblocks, int step_index, int reset_next = 0, int gated = 0);
 hipError_t launch_cont2cart_out(const Ctx &c, const double *u, const double *v, const amr_array4 &vc);
 // Conversions between Array4 views and pitched arrays, one launch for a list (the views must
-// live until it); unpack: shift (device) is subtracted
+// live until it); unpack: shift (device) is subtracted, and views that overlap are written in
+// the list's order, the last one's values staying
 constexpr int kCopyMax = 10;
 struct Copies {
     struct Item {
@@ -326,6 +327,9 @@ struct Copies {
     int count = 0;
     void face(const Ctx &c, const amr_array4 &a, const double *p, int dir);
     void cell(const Ctx &c, const amr_array4 &a, int comp, const double *p, const double *shift = nullptr);
+    // past the last item that can be written in one launch with item `first`: none of them reaches
+    // into the memory of another
+    int disjoint_end(int first) const;
 
 private:
     void add(const amr_array4 &a, int comp, const double *p, int nx, int ny, const double *shift)

@@ -783,23 +783,48 @@ void Copies::cell(const Ctx &c, const amr_array4 &a, int comp, const double *p, 
     add(a, comp, p, c.g.n, c.g.n, shift);
 }
 
-static hipError_t launch_copies(const Ctx &c, const Copies &b, void (*kern)(CopyItems, int))
+int Copies::disjoint_end(int first) const
 {
-    if (b.count == 0) return hipSuccess;
-    if (b.count > kCopyMax) return hipErrorInvalidValue;
+    uintptr_t lo[kCopyMax], hi[kCopyMax];
+    for (int q = first; q < count; ++q) {
+        const A4 a = make_a4(*it[q].a);
+        const int64_t at = a.ns * it[q].comp - a.lo0 - a.js * a.lo1;  // of cell or face (0, 0)
+        lo[q] = (uintptr_t)a.ptr + 8 * at;
+        hi[q] = lo[q] + 8 * (a.js * (it[q].ny - 1) + it[q].nx);
+        for (int r = first; r < q; ++r)
+            if (lo[q] < hi[r] && lo[r] < hi[q]) return q;
+    }
+    return count;
+}
+
+static hipError_t launch_copies(const Ctx &c, const Copies &b, int first, int end, void (*kern)(CopyItems, int))
+{
+    if (first == end) return hipSuccess;
     CopyItems t{};
     int nx = 0, ny = 0;
-    for (int q = 0; q < b.count; ++q) {
+    for (int q = first; q < end; ++q) {
         const Copies::Item &s = b.it[q];
-        t.it[q] = {make_a4(*s.a), const_cast<double *>(s.p), s.shift, s.comp, s.nx, s.ny};
+        t.it[q - first] = {make_a4(*s.a), const_cast<double *>(s.p), s.shift, s.comp, s.nx, s.ny};
         nx = std::max(nx, s.nx);
         ny = std::max(ny, s.ny);
     }
-    hipLaunchKernelGGL(kern, dim3((nx + 63) / 64, (ny + 3) / 4, b.count), dim3(256), 0, c.stream, t, c.g.P);
+    hipLaunchKernelGGL(kern, dim3((nx + 63) / 64, (ny + 3) / 4, end - first), dim3(256), 0, c.stream, t, c.g.P);
     return hipGetLastError();
 }
-hipError_t launch_pack(const Ctx &c, const Copies &b) { return launch_copies(c, b, k_pack); }
-hipError_t launch_unpack(const Ctx &c, const Copies &b) { return launch_copies(c, b, k_unpack); }
+hipError_t launch_pack(const Ctx &c, const Copies &b)
+{
+    if (b.count > kCopyMax) return hipErrorInvalidValue;
+    return launch_copies(c, b, 0, b.count, k_pack);
+}
+hipError_t launch_unpack(const Ctx &c, const Copies &b)
+{
+    if (b.count > kCopyMax) return hipErrorInvalidValue;
+    for (int first = 0, end; first < b.count; first = end) {
+        end = b.disjoint_end(first);
+        if (hipError_t e = launch_copies(c, b, first, end, k_unpack)) return e;
+    }
+    return hipSuccess;
+}
 
 hipError_t launch_unpack_cell_shift(const Ctx &c, const double *src, const amr_array4 &a, int comp,
                                     int fill_ghosts, const double *shift)
