@@ -555,9 +555,8 @@ int launch_pseudo_iteration(amressif_ctx *ctx, int it, int *nb, bool chained)
         a.uo = c.S1[0]; a.vo = c.S1[1];
         a.it = it;
         a.chained = chained;
-        // (it moves 48 B per cell: u^k, v^k, c_u, c_v in, u^{k+1}, v^{k+1} out; its record keeps the
-        // bytes of the two two-stage passes it counts as)
-        HIPCHK(amr::kprof_begin(c, amr::KP_ITER, amr::KL_MOM, it, 2 * 64.0 * (double)c.g.n * c.g.n));
+        // 48 B per cell: u^k, v^k, c_u, c_v in; u^{k+1}, v^{k+1} out
+        HIPCHK(amr::kprof_begin(c, amr::KP_ITER, amr::KL_MOM, it, 48.0 * (double)c.g.n * c.g.n));
         HIPCHK(amr::launch_iteration(c, a, nb));
         HIPCHK(amr::kprof_end(c));
         std::swap(c.U[0], c.S1[0]);
@@ -655,12 +654,9 @@ hipError_t kprof_collect(const Ctx &c)
             float ms = 0.f;
             hipError_t err = hipEventElapsedTime(&ms, r.e0, r.e1);
             if (err != hipSuccess) return err;
-            const bool both = r.id == KP_ITER;
-            for (int id = both ? KP_PAIR : r.id; id <= (both ? KP_PAIR_LAST : r.id); ++id) {
-                k->sum_ms[id] += both ? 0.5 * ms : ms;
-                k->sum_bytes[id] += both ? 0.5 * r.bytes : r.bytes;
-                k->cnt[id] += 1;
-            }
+            k->sum_ms[r.id] += ms;
+            k->sum_bytes[r.id] += r.bytes;
+            k->cnt[r.id] += 1;
         }
         k->pool.push_back(r.e0);
         k->pool.push_back(r.e1);

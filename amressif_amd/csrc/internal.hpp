@@ -105,8 +105,8 @@ enum KProfId {
     KP_PAIR,         // k_stage_pair<false>: FP64 RK stages 1-2
     KP_PAIR_LAST,    // k_stage_pair<true>: FP64 RK stages 3-4 + norm partials
     KP_MPAIR,        // k_mixed_pair: mixed residual + tangent-linear update in one pass
-    KP_COUNT,
-    KP_ITER = KP_COUNT  // k_iter_tile, all four stages: half its record to KP_PAIR, half to KP_PAIR_LAST
+    KP_ITER,         // k_iter_tile: FP64 pseudo-iteration of four stages in one pass
+    KP_COUNT
 };
 enum KProfLoop { KL_MOM = 0, KL_MG, KL_PHASE, KL_ONCE, KL_PROJ };
 struct KProf {

@@ -67,6 +67,7 @@ STEP_KERNELS = {
     "pair": ("amr::k_stage_pair<false> (FP64 RK stages 1-2 in one pass)", "pair_fp64"),
     "pair_last": ("amr::k_stage_pair<true> (FP64 RK stages 3-4 in one pass + norm partials)", None),
     "mpair": ("amr::k_mixed_pair (mixed residual + FP32 tangent-linear update in one pass)", "mpair_mixed"),
+    "iter": ("amr::k_iter_tile (FP64 pseudo-iteration of four RK stages in one pass)", None),
 }
 
 

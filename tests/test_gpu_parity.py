@@ -615,9 +615,9 @@ def test_kernel_timing_diagnostic():
     assert ms > 0 and nbytes == 2 * (1 << 24)
 
 
-@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("prec,tile", [(0, "0"), (0, "1"), (1, "1")])
 @pytest.mark.parametrize("batch", ["0", "1"])
-def test_in_step_kernel_timing_counts_and_leaves_results_unchanged(prec, batch):
+def test_in_step_kernel_timing_counts_and_leaves_results_unchanged(prec, tile, batch, monkeypatch):
     """The in-step timing hook counts exactly the launches that did work (from
     the step statistics) and does not change the step's results; with the first
     V-cycle batch capped at one cycle, the projections enqueued behind unfinished
@@ -625,6 +625,7 @@ def test_in_step_kernel_timing_counts_and_leaves_results_unchanged(prec, batch):
     import os
     api = _api()
     n, steps = 256, 4
+    monkeypatch.setenv("AMRESSIF_ITER_TILE", tile)
     state = W.initial_state(n, "seeded")
     plain = api.Run.from_numpy(api.cavity_inputs(n, 1000.0, precision=prec), state)
     plain.advance(steps)
@@ -647,8 +648,10 @@ def test_in_step_kernel_timing_counts_and_leaves_results_unchanged(prec, batch):
         assert np.array_equal(got[k], ref[k]), k
     pi = sum(s["pseudo_iters"] for s in stats)
     vc = sum(s["vcycles"] for s in stats)
+    assert t["iter"][1] == (pi if prec == 0 and tile == "1" else 0)  # all four stages in one pass
     if prec == 0:  # two stages per pass
-        assert t["pair"][1] == pi and t["pair_last"][1] == pi
+        pairs = pi if tile == "0" else 0
+        assert t["pair"][1] == pairs and t["pair_last"][1] == pairs
         assert t["stage"][1] == 0 and t["stage_last"][1] == 0
         assert t["resid"][1] == 0 and t["tangent"][1] == 0
     else:  # the mixed iteration in one pass
@@ -659,7 +662,7 @@ def test_in_step_kernel_timing_counts_and_leaves_results_unchanged(prec, batch):
     assert t["project"][1] == steps and t["poisson_start"][1] == steps
     cells = float(n * n)
     per_cell = {"stage": 64, "stage_last": 64, "resid": 48, "tangent": 48, "pair": 64, "pair_last": 64,
-                "mpair": 48}
+                "mpair": 48, "iter": 48}
     for name, (ms, cnt, nbytes) in t.items():
         assert (ms > 0) == (cnt > 0) and (nbytes > 0) == (cnt > 0), name
         assert ms < 50.0, name  # a 256^2 launch takes microseconds
