@@ -967,7 +967,7 @@ int amressif_create(const amressif_inputs *in, void *hip_stream, amressif_ctx **
                                                       "with an odd m > 2048)");
             const int bx = B.nx, by = B.ny;
             const double pi = 3.14159265358979323846;
-            c.big_strip = amr::bottom_strips(bx, by);
+            c.big_strip = amr::bottom_strips(bx, by, in->precision == AMRESSIF_MIXED);
             const int lx = c.big_strip ? (int)round_up(bx, 128) : bx, ly = c.big_strip ? (int)round_up(by, 128) : by;
             // C_x, C_y and D+; strip-wise also C_x^T and C_y^T, all padded with zeros
             std::vector<double> tab((c.big_strip ? 2 : 1) * ((size_t)lx * lx + (size_t)ly * ly) + (size_t)ly * lx);

@@ -303,7 +303,7 @@ hipError_t launch_mg_start(const Ctx &c, int require_mom = 0, const double *us =
 hipError_t launch_poisson_start(const Ctx &c, int mode, int center, const double *phi1, const double *phi2,
                                 double *phi0, int mixed, const double *us = nullptr, const double *vs = nullptr);
 hipError_t launch_fin_resid(const Ctx &c, int nblocks);
-bool bottom_strips(int nx, int ny);  // a dense bottom level solved strip-wise
+bool bottom_strips(int nx, int ny, bool mixed);  // a dense bottom level solved strip-wise
 hipError_t launch_vcycle(const Ctx &c, int mixed);
 hipError_t launch_vcycle_step(const Ctx &c, int mixed, int par, const double *phi_in, double *phi_out, int *nblocks);
 hipError_t launch_correct_residual(const Ctx &c, const double *phi_in, double *phi_out, int with_correction,

@@ -1787,9 +1787,6 @@ __global__ __launch_bounds__(256) void k_dense_mm(const T *A, int lda, int ta, c
 // products (a strip per workgroup in LDS, a 16-row tile per wave) and a second one
 // multiplies by C_x^T (a tile per wave).  Latency bound: a tile's whole depth, 128, is
 // loaded at once.  At 125^2 in FP32 12.0 + 4.1 us against 4 x 7.1, in FP64 18.6 + 6.5.
-// Past 128 a strip's products take several rounds of loads on few workgroups: with a
-// limit of 256 they took 34 us (FP32) and 52 (FP64) at 191^2 and would at 129^2, where four
-// dense products take about 29.
 constexpr int kStripLd = 16;   // row stride of a strip: four rows of 16 lanes in different banks
 constexpr int kStripWaves = 8;
 constexpr int kStripMax = 128;
@@ -1938,7 +1935,16 @@ __global__ __launch_bounds__(64) void k_dense_last(const T *WT, const T *CxT, T 
 }
 
 static int round_up128(int n) { return (n + 127) / 128 * 128; }
-bool bottom_strips(int nx, int ny) { return nx <= kStripMax && ny <= kStripMax; }
+// A strip's products have the depth of 128 cells whatever the side.  In FP32 they are ahead from the
+// smallest level on (a solve at 66^2, bottom 33^2, in 302 us against 313; 254^2 in 320 against 400).  In
+// FP64 up to 63 cells the four dense products are, a block or less of k each (66^2: 409 us against 441,
+// 98^2: 431 against 446, 126^2: 434 against 450), and the strips from 65 on (130^2: 452 against 461, 162^2:
+// 457 against 487).  Past 128 the strips take several rounds of loads on few workgroups: 34 us
+// (FP32) and 52 (FP64) at 191^2, and would at 129^2, where four dense products take about 29.
+bool bottom_strips(int nx, int ny, bool mixed)
+{
+    return std::max(nx, ny) <= kStripMax && (mixed || std::min(nx, ny) >= 64);
+}
 
 template <class T>
 static hipError_t dense_bottom(const Ctx &c, const T *r, int pr, T *e, int pe, const Level &L)

@@ -502,11 +502,12 @@ def test_odd_bottom_poisson_solve_matches_the_exact_solve(n):
         assert rel(sol.cpu().numpy()[1:-1, 1:-1], xe[1:-1, 1:-1]) < bar, prec
 
 
-@pytest.mark.parametrize("n", [66, 70, 162, 226, 254, 258])
+@pytest.mark.parametrize("n", [66, 70, 126, 130, 162, 226, 254, 258])
 def test_odd_bottom_strips_match_the_exact_solve(n):
-    """Odd bottoms of 33, 35, 81, 113, 127 and 129 cells a side: one past two
-    whole 16-column strips, the row tiles' remainders, the last size solved strip
-    by strip and the first one solved by four dense products, in both types."""
+    """Odd bottoms of 33, 35, 63, 65, 81, 113, 127 and 129 cells a side in both types:
+    one past two whole 16-column strips (FP32; FP64 takes strips from 65 on and
+    four dense products below), the row tiles' remainders, the last size solved
+    strip by strip and the first one past it."""
     api = _api()
     rng = np.random.default_rng(n)
     rhs = np.zeros((n + 2, n + 2))

@@ -55,6 +55,17 @@ def test_timing_the_one_launch_pseudo_iteration_and_its_refusal():
         api.Context(api.cavity_inputs(10240, 400.0)).time_kernel(11, reps=3)
 
 
+def test_odd_bottoms_are_solved_by_the_faster_form(tmp_path):
+    """Strips of a padded depth of 128 or four dense products: FP64 takes the
+    products up to 63 cells a side, where they are faster, and both types past
+    128."""
+    out = _run(tmp_path, """
+    for (int m : {33, 49, 63, 65, 81, 127, 129})
+        std::printf("%d%d ", (int)amr::bottom_strips(m, m, false), (int)amr::bottom_strips(m, m, true));
+    """)
+    assert out == ["01", "01", "01", "11", "11", "11", "00"]
+
+
 def test_overlapping_output_views_are_not_written_in_one_launch(tmp_path):
     """Items that share memory start a new launch, so the last one of the list
     stays, as with a launch each: two views of one array, a view into the end of
