@@ -971,18 +971,23 @@ int amressif_create(const amressif_inputs *in, void *hip_stream, amressif_ctx **
             const int lx = c.big_strip ? (int)round_up(bx, 128) : bx, ly = c.big_strip ? (int)round_up(by, 128) : by;
             // C_x, C_y and D+; strip-wise also C_x^T and C_y^T, all padded with zeros
             std::vector<double> tab((c.big_strip ? 2 : 1) * ((size_t)lx * lx + (size_t)ly * ly) + (size_t)ly * lx);
-            double *at = tab.data();
-            auto fill = [&](int m, int ld, bool transposed) {
+            double *at = tab.data(), *Cx = at;
+            auto fill = [&](int m, int ld) {  // C, and C^T after it
+                const double s0 = std::sqrt(1.0 / m), s1 = std::sqrt(2.0 / m);
+                if (at != Cx && m == bx && ld == lx) std::copy(Cx, Cx + (size_t)ld * ld, at);  // (the cosines are most of the set-up)
+                else
+                    for (int i = 0; i < m; ++i)
+                        for (int k = 0; k < m; ++k)
+                            at[(size_t)i * ld + k] = (k == 0 ? s0 : s1) * std::cos(pi * k * (2 * i + 1) / (2.0 * m));
+                double *C = at;
+                at += (size_t)ld * ld;
+                if (!c.big_strip) return;
                 for (int i = 0; i < m; ++i)
-                    for (int k = 0; k < m; ++k)
-                        at[transposed ? (size_t)k * ld + i : (size_t)i * ld + k] =
-                            std::sqrt((k == 0 ? 1.0 : 2.0) / m) * std::cos(pi * k * (2 * i + 1) / (2.0 * m));
+                    for (int k = 0; k < m; ++k) at[(size_t)k * ld + i] = C[(size_t)i * ld + k];
                 at += (size_t)ld * ld;
             };
-            fill(bx, lx, false);
-            if (c.big_strip) fill(bx, lx, true);
-            fill(by, ly, false);
-            if (c.big_strip) fill(by, ly, true);
+            fill(bx, lx);
+            fill(by, ly);
             double *Dinv = at;
             for (int mm = 0; mm < by; ++mm)
                 for (int k = 0; k < bx; ++k) {
