@@ -272,12 +272,12 @@ __global__ __launch_bounds__(1024) void k_gen_leg3(Geom g, Level F, Level Cl, in
     double hlo[2] = {0.0, 0.0}, hhi[2] = {0.0, 0.0}, acc = 0.0;
     load(F.r, ps, nr);
     if (UP) {
-        load(F.e, ps, ne);
-        load_coarse((ps >> 1) - ((ps & 1) ? 0 : 1));
+        load(F.e, ps, ne);  // ps is even, as zc is
+        load_coarse((ps >> 1) - 1);
         rows_of(hlo);
-        load_coarse((ps >> 1) + ((ps & 1) ? 1 : 0));
+        load_coarse(ps >> 1);
         rows_of(hhi);
-        if (!(ps & 1)) load_coarse((ps >> 1) + 1);
+        load_coarse((ps >> 1) + 1);
     }
     __syncthreads();
     int bf = 0;
@@ -524,7 +524,8 @@ __global__ __launch_bounds__(1024) void k_gen_fin_outer(const double *partials, 
 // 128^3, 25 at 72^3, 23 at 64^3, 22 at 32^3 against 1218, 153, 31, 23 and 14 of the tiles
 static bool leg_march(int n) { return n > 64; }
 
-// Planes per workgroup of k_gen_leg3 (even): the shortest rounds of 256 workgroups, each of
+// Planes per workgroup of k_gen_leg3 (even: a coarse plane's two children are one workgroup's,
+// and the march up starts on an even plane): the shortest rounds of 256 workgroups, each of
 // zc planes and about nine to fill and drain the half-sweeps
 static int leg_chunk(int n, int tiles)
 {
@@ -540,11 +541,12 @@ static int leg_chunk(int n, int tiles)
 hipError_t vcycle(const Ctx &c, hipStream_t s, const Ctl *ctl)
 {
     const int L = c.nlev;
-    auto leg = [&](int l, bool up) {
+    auto leg = [&](int l, bool up) -> hipError_t {
         const Level &F = c.lev[l], &Cl = c.lev[l + 1];
         if (c.g.dim == 3 && leg_march(F.n)) {
             const int h = up ? 4 : 6, ntx = (F.n + 63 - 2 * h) / (64 - 2 * h), nty = (F.n + 31 - 2 * h) / (32 - 2 * h);
             const int zc = leg_chunk(F.n, ntx * nty);
+            if (zc & 1) return hipErrorInvalidValue;
             const dim3 grid(ntx * nty * ((F.n + zc - 1) / zc)), block(1024);
             if (up) hipLaunchKernelGGL(k_gen_leg3<true>, grid, block, 0, s, c.g, F, Cl, ntx, nty, zc, ctl);
             else hipLaunchKernelGGL(k_gen_leg3<false>, grid, block, 0, s, c.g, F, Cl, ntx, nty, zc, ctl);
@@ -559,13 +561,16 @@ hipError_t vcycle(const Ctx &c, hipStream_t s, const Ctl *ctl)
             if (up) hipLaunchKernelGGL((k_gen_leg<2, true>), grid, block, 0, s, c.g, F, Cl, nt, ctl);
             else hipLaunchKernelGGL((k_gen_leg<2, false>), grid, block, 0, s, c.g, F, Cl, nt, ctl);
         }
+        return hipGetLastError();
     };
-    for (int l = 0; l + 1 < L; ++l) leg(l, false);
+    for (int l = 0; l + 1 < L; ++l)
+        if (hipError_t e = leg(l, false)) return e;
     const Level &B = c.lev[L - 1];
     if (c.g.dim == 3) hipLaunchKernelGGL(k_gen_exact3, dim3(1), dim3(1024), 0, s, B.r, B.out, B.n, c.exact, ctl);
     else if (hipError_t e = launch_exact2(s, B.r, B.out, B.n, c.exact, ctl)) return e;
-    for (int l = L - 2; l >= 0; --l) leg(l, true);
-    return hipGetLastError();
+    for (int l = L - 2; l >= 0; --l)
+        if (hipError_t e = leg(l, true)) return e;
+    return hipSuccess;
 }
 
 static int outer_chunk(int dim, int n) { return dim == 3 ? (n >= 128 ? 16 : 4) : (n >= 1024 ? 8 : 2); }
