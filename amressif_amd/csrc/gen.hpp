@@ -68,7 +68,7 @@ struct Ctx {
 
 // ---- launchers (kernels_gen.hip); every guarded kernel returns at once once
 // its loop's flag in the control block is set
-hipError_t cells(const Ctx &c, hipStream_t s, double *const *faces, double *X, const Ctl *guard);
+hipError_t cells(const Ctx &c, hipStream_t s, double *const *faces, double *X);
 // 2D: the step's pseudo-iteration `it` (or the explicit update), out <- the last stage from base, with its norm
 // partials; chained: it also takes the norm of the launch before and ends the loop
 hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, int it, bool chained,

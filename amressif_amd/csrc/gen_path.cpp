@@ -359,7 +359,7 @@ int amr_gen_store_state(amressif_ctx *ctx, amr_array4 *vel, amr_array4 *velPrev,
             if ((d < g.dim && (velCart->lo[d] < -2 || velCart->hi[d] > g.n + 1)) ||
                 (d >= g.dim && (velCart->lo[d] != 0 || velCart->hi[d] != 0)))
                 return gfail(ctx, AMRESSIF_ERR_ARG, "velCart: at most two ghost layers");
-        GCHK(G::cells(gc, c.stream, gc.U, gc.X, nullptr));
+        GCHK(G::cells(gc, c.stream, gc.U, gc.X));
         GCHK(G::unpack_velcart(gc, c.stream, gc.X, *velCart));
     }
     GCHK(hipStreamSynchronize(c.stream));
@@ -501,7 +501,7 @@ int amr_gen_store_state_mf(amressif_ctx *ctx, amr_multifab *vel, amr_multifab *v
         }
     }
     if (velCart) {
-        GCHK(G::cells(gc, c.stream, gc.U, gc.X, nullptr));
+        GCHK(G::cells(gc, c.stream, gc.U, gc.X));
         for (int b = 0; b < velCart->nbox; ++b) GCHK(G::unpack_velcart(gc, c.stream, gc.X, velCart->fab[b]));
     }
     GCHK(hipStreamSynchronize(c.stream));
@@ -641,7 +641,7 @@ int amr_gen_time_kernel(amressif_ctx *ctx, int which, int reps, double *avg_ms, 
         GCHK(hipMemcpyAsync(gc.B[d], gc.U[d], g.nf[d] * 8, hipMemcpyDeviceToDevice, c.stream));
     GCHK(G::bdf2(gc, c.stream));
     auto launch = [&]() -> hipError_t {
-        if (which == 0) return G::cells(gc, c.stream, gc.U, gc.X, nullptr);
+        if (which == 0) return G::cells(gc, c.stream, gc.U, gc.X);
         if (g.dim == 3) return G::stage3(gc, c.stream, gc.U, gc.B, gc.S, gc.rk[0], which == 2, nullptr);
         return G::iteration2(gc, c.stream, gc.B, gc.S, 0, false, nullptr);
     };

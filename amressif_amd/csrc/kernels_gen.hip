@@ -71,9 +71,8 @@ __device__ __forceinline__ void wall_rule(const Geom &g, int kind, int d, double
 
 // ------------------------------------------------------------ cell velocities
 __global__ __launch_bounds__(B) void k_gen_cells(Geom g, const double *f0, const double *f1, const double *f2,
-                                                 double *X, const Ctl *guard)
+                                                 double *X)
 {
-    if (guard && guard->mom_done) return;
     const int64_t s = g.n + 4, sk = g.dim == 3 ? s : 1;
     const int64_t q = gid();
     if (q >= s * s * sk) return;
@@ -788,10 +787,9 @@ inline int nblk(int64_t m) { return (int)((m + B - 1) / B); }
 }  // namespace
 
 // ============================================================ launchers
-hipError_t cells(const Ctx &c, hipStream_t s, double *const *f, double *X, const Ctl *guard)
+hipError_t cells(const Ctx &c, hipStream_t s, double *const *f, double *X)
 {
-    hipLaunchKernelGGL(k_gen_cells, dim3(nblk(c.g.xs)), dim3(B), 0, s, c.g, f[0], f[1], c.g.dim == 3 ? f[2] : f[0],
-                       X, guard);
+    hipLaunchKernelGGL(k_gen_cells, dim3(nblk(c.g.xs)), dim3(B), 0, s, c.g, f[0], f[1], c.g.dim == 3 ? f[2] : f[0], X);
     return hipGetLastError();
 }
 
