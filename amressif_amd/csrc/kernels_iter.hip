@@ -271,7 +271,7 @@ __global__ __launch_bounds__(64 * kItW) void k_iter_tile(IterTile a)
 // Rows per thread.  A round of 256 workgroups takes about 1.5 us per row held plus 5,
 // over a launch's 6 us (128^2: 17.6, 24.0 and 29.8 us with 4, 6 and 8 rows), and a
 // tile writes 8, 24 and 40 rows of its 32, 48 and 64: the height whose rounds are
-// shortest, 4 up to n = 279, 6 to 439, mostly 8 above.  (Sixteen waves of half the
+// shortest, 4 up to n = 279, 6 to 479 and from 640 to 679, 8 elsewhere.  (Sixteen waves of half the
 // rows each are no faster: 24.2 us for 48 rows, 33.6 for 64.)
 int rows_per_thread(int n)
 {

@@ -118,11 +118,12 @@ def test_2d_periodic_steps_match_oracle(bc_lo, bc_hi):
     _check(ref, ref_stats, got, stats, 2)
 
 
-@pytest.mark.parametrize("n", [4, 5, 24, 31, 288])
+@pytest.mark.parametrize("n", [4, 5, 24, 31, 288, 480])
 @pytest.mark.parametrize("bc_lo,bc_hi", [((111, 111, 0), (111, 111, 0)), ((-135, 111, 0), (165, 111, 0))])
 def test_2d_pseudo_iteration_tile_edges(n, bc_lo, bc_hi):
     """The one-launch 2D pseudo-iteration where its halo of 12 wraps a small
-    periodic box several times, and in the 40-row tiles (n >= 280)."""
+    periodic box several times, in the tiles of 8 rows (n <= 279), of 24 (288)
+    and of 40 (480, one face past twelve of them)."""
     ref, ref_stats, got, stats, _, _ = _run_pair(2, n, 300.0, bc_lo, bc_hi, 2, inflow=(0.5, -0.2, 0.0), amp=0.1)
     _check(ref, ref_stats, got, stats, 2)
 
@@ -164,6 +165,15 @@ def test_3d_stage_kernel_tile_edges(n, bc_lo, bc_hi):
     one tile, whole tiles of rows (n + 1 = 11, 33), one row past (n + 1 = 5, 21), the last size of one
     column tile (n + 1 = 57) and the first of two."""
     ref, ref_stats, got, stats, _, _ = _run_pair(3, n, 150.0, bc_lo, bc_hi, 2, inflow=(0.4, 0.2, -0.3), amp=0.1)
+    _check(ref, ref_stats, got, stats, 3)
+
+
+@pytest.mark.parametrize("zc", ["1", "2", "7", "1000"])
+def test_3d_stage_kernel_planes_per_workgroup(zc, monkeypatch):
+    """The one-pass 3D stage with chunks of one plane, two, a number that leaves
+    a remainder, and the whole march in one workgroup."""
+    monkeypatch.setenv("AMRESSIF_GEN_S3ZC", zc)
+    ref, ref_stats, got, stats, _, _ = _run_pair(3, 20, 150.0, (111, 135, 135), (111, 165, -135), 2, amp=0.1)
     _check(ref, ref_stats, got, stats, 3)
 
 

@@ -321,13 +321,14 @@ def test_two_stage_pass_matches_four_stage_launches(n, rows, init, bc, lid):
 @pytest.mark.parametrize("n,init,bc,lid", [
     (4, "seeded", 0, False), (8, "seeded", 3, False), (38, "seeded", 1, False), (40, "seeded", 2, False),
     (78, "zero", 0, True), (128, "seeded", 2, True), (279, "seeded", 0, True), (280, "seeded", 1, False),
-    (319, "seeded", 2, True), (320, "seeded", 3, False), (600, "seeded", 0, False)])
+    (319, "seeded", 2, True), (320, "seeded", 3, False), (479, "seeded", 3, False), (480, "seeded", 2, True),
+    (600, "seeded", 0, False)])
 def test_one_launch_pseudo_iteration_matches_four_stage_launches(n, init, bc, lid):
     """The FP64 pseudo-iteration as one tile launch against four single-stage
     launches: the same pseudo-iteration counts and the same fields to rounding,
-    below one tile (40 columns), at whole tiles (n + 1 = 80, 280, 320) and one
-    face past them, in the 8-row tiles (n <= 279) and the 40-row ones, with
-    every wall set, a lid profile, and batches that overshoot convergence (the
+    below one tile (40 columns), at whole tiles (n + 1 = 80, 280, 320, 480) and
+    one face past them, in the tiles of 8 rows (n <= 279), of 24 (to 479) and of
+    40 (480, 600), with every wall set, a lid profile, and batches that overshoot convergence (the
     skipped launches copy the base)."""
     api = _api()
     prof = W.lid_profile(n) if lid else None
@@ -353,7 +354,7 @@ def test_one_launch_pseudo_iteration_matches_four_stage_launches(n, init, bc, li
     assert rel(p1 - p1.mean(), p4 - p4.mean()) < 1e-11
 
 
-@pytest.mark.parametrize("n", [40, 320])
+@pytest.mark.parametrize("n", [40, 320, 500])
 @pytest.mark.parametrize("end", ["cap", "diverged", "nonfinite"])
 def test_one_launch_pseudo_iteration_ends_the_loop_like_its_finalizer(n, end):
     """A tile launch takes the norm of the launch before it and ends the loop
