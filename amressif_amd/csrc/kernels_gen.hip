@@ -135,10 +135,12 @@ __device__ __forceinline__ double face_flux(const FaceVel &f, double xm, double 
 // u* <- u^k + rk (R(u*) - (1.5/dt) u* + C) on every face, from the faces
 // alone: 96 B per cell (u*, u^k and C in, the new u* out; 72 B where u* is
 // u^k), where the three passes it replaces (cell velocities, fluxTotal, update)
-// moved 2.4 times that.  At 256^3 a launch takes 439 us (3.7 TB/s; with the norm
-// partials 449) against 162 + 390 + 374 us of the three passes, at 144^3 88 us
-// against 34 + 69 + 60, at 64^3 22 against 5.5 + 22 + 7.  Bound by the arithmetic
-// of a plane (2.7 us, about 60% of it in the FP64 pipe) more than by memory.
+// moved 2.4 times that.  At 256^3 a launch takes 426 us (with the norm partials 445)
+// against 162 + 390 + 374 us of the three passes, at 144^3 77 us against 34 + 69 +
+// 60, at 64^3 22 against 5.5 + 22 + 7.  Bound by memory at 256^3: the counters give
+// 1.36 GB read and 0.43 written (1.62 GB without the halo), 4.2 TB/s where a large
+// copy reaches 4.9, with the VALU busy 38% of the time (FP64 instructions 20%); on
+// small grids by a plane's chain and the planes of prologue.
 //
 // A workgroup owns 58 columns x kS3Y rows and marches up a chunk of planes.  Wave r
 // works on rows y0 - 3 + 2 r and the next, lane l on column x0 - 3 + l, so the

@@ -178,10 +178,14 @@ __global__ __launch_bounds__(LegShape<DIM>::NT) void k_gen_leg(Geom g, Level F, 
 // neighbours are the thread's other row or, published a step before, the next wave's
 // row in LDS: one barrier per plane.  Outside a wall the loads give 0 and 1/diag is 0,
 // so nothing moves there.  Halos: 4 rings for four half-sweeps; going down one more for
-// the residual and one to start on even cells.  Each plane is read once: 16 B per
-// cell down, 24 B up (where five launches moved about 140): 163 us at 256^3 against 477
-// down and 527 up.  Bound by the arithmetic of a plane (1.5 us) with half the lanes
-// idle in each half-sweep.
+// the residual and one to start on even cells.  A workgroup loads each plane of its
+// tile once: 17 B per cell down, 25 up (coarse cells with them) are what a leg cannot
+// do without.  The halo's loads are 1.97 times that down and 1.52 up, plus nine and
+// seven planes a chunk, most of them from the L2: the counters give 20 and 28 B (five
+// launches moved about 140).  163 us a leg at 256^3 against 477 down and 527 up, at 2.1
+// and 2.9 TB/s.  Bound by the instructions of a plane (1.7 us; where a workgroup runs
+// the VALU is busy 77% of the time down, 65% up) with half the lanes idle in each
+// half-sweep.
 template <bool UP>
 __global__ __launch_bounds__(1024) void k_gen_leg3(Geom g, Level F, Level Cl, int ntx, int nty, int zc, const Ctl *ctl)
 {

@@ -170,7 +170,8 @@ typedef struct {
 
 /* amressif_load_state over several boxes: each box's valid region is
  * gathered into the context's one-box working set (a shared face is read
- * from the later box; a consistent MultiFab holds the same value in both).
+ * from the later box; a consistent MultiFab holds the same value in both, as
+ * on faces 0 and n of a periodic direction).
  * userCtx may be NULL (p = phi = 0).  2D and 3D, walls and periodic
  * directions; boxes are validated before the first copy, so a refused load
  * leaves the state as it was. */
