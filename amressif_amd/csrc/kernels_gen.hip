@@ -816,7 +816,9 @@ int stage3_blocks(const Ctx &c)
     return c.s3_ntx * c.s3_nty * ((c.g.n + 1 + c.s3_zc - 1) / c.s3_zc);
 }
 
-// 2D: two sets of norm records in turn (a launch reads the one before's while it writes its own)
+// 2D: a pseudo-iteration is one tile launch at every size: 17 us at 384^2, 56 at 1024^2, 200 at
+// 2048^2 and 780 at 4096^2, where four stages of three passes each took 48, 131, 409 and 2300.
+// Two sets of norm records in turn (a launch reads the one before's while it writes its own).
 static double *records2(const Ctx &c, int it) { return c.partials + (it & 1) * 3 * (int64_t)iter_tile_blocks(c.g.n); }
 
 hipError_t iteration2(const Ctx &c, hipStream_t s, double *const *base, double *const *out, int it, bool chained,
