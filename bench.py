@@ -109,10 +109,10 @@ def read_traffic(kernel_key: str):
     return vals.get(key)
 
 
-def step_bytes_fp64(n, pseudo_iters, vcycles, stage_passes=4):
+def step_bytes_fp64(n, pseudo_iters, vcycles, pseudo_bytes=4 * 64):
     """Algorithmic HBM bytes of one FP64 step at n^2 cells, kernel by kernel:
-    per pseudo-iteration `stage_passes` passes of 64 B/cell (4: one per RK4
-    stage; 2: two stages per pass, the first kept in registers; the pressure
+    `pseudo_bytes` per cell and pseudo-iteration (four passes of 64 B, one per RK4
+    stage; two, the first stage of each kept in registers; one of 48 B; the pressure
     gradient sits in the BDF2 constant, put there by the previous projection); per V-cycle the
     finest down-leg smoother with the fused restriction (r in, e out, coarse
     r out: 18 B), the finest up-leg smoother with the fused FP64 outer step
@@ -123,7 +123,7 @@ def step_bytes_fp64(n, pseudo_iters, vcycles, stage_passes=4):
     the next step's BDF2 constant (u*, v*, phi, p, u^n in; u, v, p, c and the
     copy of u out: 104 B)."""
     cells = float(n) * n
-    return cells * (pseudo_iters * stage_passes * 64 + vcycles * (18 + 50 + 44 / 3) + 40 + 104)
+    return cells * (pseudo_iters * pseudo_bytes + vcycles * (18 + 50 + 44 / 3) + 40 + 104)
 
 
 def run_precision(api, W, n, ren, precision, state, warmup, steps, torch):
@@ -318,15 +318,20 @@ def main():
         o = out["fp64"]
         sec = o["ms_per_step"] * 1e-3
         nbytes = step_bytes_fp64(n, o["pseudo_iters"], o["vcycles"])
-        paired = any(r["kernel"].startswith("amr::k_stage_pair") for r in kernels.get("fp64", []))
-        nb2 = step_bytes_fp64(n, o["pseudo_iters"], o["vcycles"], 2) if paired else nbytes
+        ran = [r["kernel"] for r in kernels.get("fp64", [])]
+        per_iter, model = 4 * 64, "as above"
+        if any(k.startswith("amr::k_stage_pair") for k in ran):
+            per_iter, model = 2 * 64, ("two passes of 64 B/cell per pseudo-iteration (k_stage_pair: the first stage "
+                                       "of each pair stays in registers)")
+        elif any(k.startswith("amr::k_iter_tile") for k in ran):
+            per_iter, model = 48, "one pass of 48 B/cell per pseudo-iteration (k_iter_tile: all four stages in registers)"
+        nb2 = step_bytes_fp64(n, o["pseudo_iters"], o["vcycles"], per_iter)
         extra["fp64_step_roofline"] = {
             "bytes_per_step": nbytes, "achieved": nbytes / sec / 1e9, "unit": "GB/s", "frac": nbytes / sec / HBM_PEAK,
             "byte_model": "four RK4 stage passes of 64 B/cell per pseudo-iteration (the minimum traffic of "
                           "one-stage-per-pass kernels)",
             "bytes_per_step_as_run": nb2, "achieved_as_run": nb2 / sec / 1e9, "frac_as_run": nb2 / sec / HBM_PEAK,
-            "byte_model_as_run": ("two passes of 64 B/cell per pseudo-iteration (k_stage_pair: the first stage "
-                                  "of each pair stays in registers)" if paired else "as above")}
+            "byte_model_as_run": model}
 
     adj = None
     if args.adjoint_n > 0 and not args.profile_run:
